@@ -147,7 +147,7 @@ struct MuyoDecoder
     uint16_t* pAttnLo = nullptr;
     uint16_t* pActHi = nullptr;  // [rows][ffn] swiglu output
     uint16_t* pActLo = nullptr;
-    float* pPartial = nullptr;   // [kMaxGemmSplits][rows][max(qkv rows, hidden)] K-split partial sums
+    float* pPartial = nullptr;   // [splits][rows][max(qkv rows, hidden)] K-split partial sums
     size_t pPartialFloats = 0;  // (or the split attention's partials, when larger)
 
     template <typename T>
@@ -1167,7 +1167,8 @@ int EnsurePrefill(MuyoDecoder* d)
     const size_t actLo = place(rows * c.feedForward * 2);
     // K-split partial sums of the GEMMs whose tiles alone leave the chip idle (GemmSplits), and,
     // between the q|k|v and o_proj GEMMs, the split attention's key-chunk partials.
-    const size_t partialFloats = std::max(kMaxGemmSplits * rows * std::max<size_t>(qkvRows, c.hidden),
+    const size_t partialFloats = std::max(GemmPartialFloats(static_cast<uint32_t>(rows),
+                                                            static_cast<uint32_t>(std::max<size_t>(qkvRows, c.hidden))),
                                           PrefillAttentionWorkspaceFloats(static_cast<uint32_t>(rows), c.heads,
                                                                           c.headDim));
     const size_t partial = place(partialFloats * 4);

@@ -1,52 +1,18 @@
-// Batched-prefill kernels for gfx950: split-f16 GEMMs on v_mfma_f32_32x32x16_f16 with fused
-// epilogues, a causal flash attention over the fp16 cache, and the row-wise glue (embedding,
-// rms_norm into split planes, rope + cache append).
-//
-// Matrix-core lane layout of v_mfma_f32_32x32x16_f16 (D = A.B, A 32x16, B 16x32), as used below:
-// lane l supplies A[l % 32][8 * (l / 32) .. +8] and B[8 * (l / 32) .. +8][l % 32], and receives
-// D[8 * (r / 4) + 4 * (l / 32) + r % 4][l % 32] in accumulator r (0..15).
+// Batched-prefill kernels for gfx950: a causal flash attention over the fp16 cache and the row-wise
+// glue (embedding, rms_norm into split planes, rope + cache append). The GEMMs are in
+// prefill_gemm.hip.
 #include <algorithm>
 #include <cmath>
 #include <initializer_list>
 #include <type_traits>
 
-#include "common.hpp"
 #include "prefill.hpp"
+#include "prefill_core.hpp"
 
 namespace muyo
 {
 namespace
 {
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef _Float16 half4 __attribute__((ext_vector_type(4)));
-typedef uint16_t ushort4v __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ floatx16 Mfma(half8 a, half8 b, floatx16 c)
-{
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
-
-/// v = hi + lo to ~21 bits. hi is v with its 13 low mantissa bits cleared: 11 significant bits,
-/// exact in f16. Rounding hi to f16 instead is not safe here: with contraction the compiler feeds
-/// a product straight into v_fma_mix*_f16 (one rounding to f16) for one use and rounds it to f32
-/// first (two roundings) for another, so the stored hi and the hi subtracted for lo can differ by
-/// an f16 ulp near a tie. The bit mask works on the f32 value, and lo = v - hi is exact in f32
-/// before its one rounding into f16. |v| must stay below 65536 (f16's range).
-__device__ __forceinline__ float HiPart(float v) { return __uint_as_float(__float_as_uint(v) & 0xFFFFE000u); }
-
-__device__ __forceinline__ _Float16 HiHalf(float v) { return static_cast<_Float16>(HiPart(v)); }
-
-__device__ __forceinline__ _Float16 LoHalf(float v) { return static_cast<_Float16>(v - HiPart(v)); }
-
-__device__ __forceinline__ void StoreSplit4(uint16_t* hi, uint16_t* lo, uint64_t at, float a, float b, float c,
-                                            float d)
-{
-    const half4 h = {HiHalf(a), HiHalf(b), HiHalf(c), HiHalf(d)};
-    const half4 l = {LoHalf(a), LoHalf(b), LoHalf(c), LoHalf(d)};
-    *reinterpret_cast<half4*>(hi + at) = h;
-    *reinterpret_cast<half4*>(lo + at) = l;
-}
-
 // ------------------------------------------------------------------------------------------------
 // Row-wise glue.
 
@@ -145,11 +111,11 @@ __global__ __launch_bounds__(256) void RmsNormSplitKernel(float* __restrict__ x,
 }
 
 /// RmsNormSplitKernel with kT threads per row (one wave, or the whole 256-thread workgroup) and
-/// at most kChunks 16-byte chunks of the row per thread, all requested before the first is used:
+/// at most kChunks 16-byte chunks of the row per thread (and kParts K splits), all requested before the first is used:
 /// every K split's part, the residual and the weight in one round of loads instead of one round
 /// per chunk. The sums run in SplitSum::At's order; the sum of squares meets across the row's
 /// waves in LDS.
-template <int kT>
+template <int kT, uint32_t kParts>
 __global__ __launch_bounds__(256) void RmsNormSplitRowsKernel(float* __restrict__ x, const float* __restrict__ w,
                                                               uint32_t rows, uint32_t cols, float eps,
                                                               uint16_t* __restrict__ hi, uint16_t* __restrict__ lo,
@@ -164,7 +130,7 @@ __global__ __launch_bounds__(256) void RmsNormSplitRowsKernel(float* __restrict_
     const bool live = row < rows;
     const uint64_t base = static_cast<uint64_t>(live ? row : 0) * cols;
     float4 v[kChunks];
-    float4 part[kMaxGemmSplits - 1][kChunks];
+    float4 part[kParts - 1][kChunks];
     float4 res[kChunks];
     float4 g[kChunks];
 #pragma unroll
@@ -175,7 +141,7 @@ __global__ __launch_bounds__(256) void RmsNormSplitRowsKernel(float* __restrict_
         const uint64_t at = base + (in ? i : 0);
         v[c] = *reinterpret_cast<const float4*>((sum.splits > 0 ? sum.partial : x) + at);
 #pragma unroll
-        for (uint32_t z = 1; z < kMaxGemmSplits; ++z)
+        for (uint32_t z = 1; z < kParts; ++z)
         {
             if (z < sum.splits)
             {
@@ -199,7 +165,7 @@ __global__ __launch_bounds__(256) void RmsNormSplitRowsKernel(float* __restrict_
         if (sum.splits > 0)
         {
 #pragma unroll
-            for (uint32_t z = 1; z < kMaxGemmSplits; ++z)
+            for (uint32_t z = 1; z < kParts; ++z)
             {
                 if (z < sum.splits)
                 {
@@ -262,19 +228,22 @@ __global__ __launch_bounds__(256) void RmsNormSplitRowsKernel(float* __restrict_
 }
 
 /// The row kernel for `cols`: a wave per row up to 1024 columns, the workgroup per row up to 4096,
-/// else the loop kernel.
+/// else the loop kernel. Sums of up to four parts keep their own kernel: the registers that eight
+/// parts take halve the waves in flight.
 hipError_t LaunchRmsNormSplitRows(hipStream_t s, float* x, const float* w, uint32_t rows, uint32_t cols, float eps,
                                   uint16_t* hi, uint16_t* lo, const SplitSum& sum)
 {
+    static_assert(kMaxGemmSplits == 8, "parts");
+    const bool few = sum.splits <= 4;
     if (cols <= 4 * 4 * kWave)
     {
-        hipLaunchKernelGGL(RmsNormSplitRowsKernel<kWave>, dim3(CeilDiv(rows, 4)), dim3(256), 0, s, x, w, rows, cols,
-                           eps, hi, lo, sum);
+        hipLaunchKernelGGL((few ? RmsNormSplitRowsKernel<kWave, 4> : RmsNormSplitRowsKernel<kWave, 8>),
+                           dim3(CeilDiv(rows, 4)), dim3(256), 0, s, x, w, rows, cols, eps, hi, lo, sum);
     }
     else if (cols <= 4 * 4 * 256)
     {
-        hipLaunchKernelGGL(RmsNormSplitRowsKernel<256>, dim3(rows), dim3(256), 0, s, x, w, rows, cols, eps, hi, lo,
-                           sum);
+        hipLaunchKernelGGL((few ? RmsNormSplitRowsKernel<256, 4> : RmsNormSplitRowsKernel<256, 8>), dim3(rows),
+                           dim3(256), 0, s, x, w, rows, cols, eps, hi, lo, sum);
     }
     else
     {
@@ -402,15 +371,42 @@ __global__ __launch_bounds__(256) void RopeSplitAppendQuadKernel(const float* __
     const uint32_t width = (heads + 2 * kvHeads) * headDim;
     const float* row = qkv + static_cast<uint64_t>(m) * width;
     const uint64_t stride = static_cast<uint64_t>(rows) * width;
-    auto value4 = [&](uint32_t col) {
-        float4v a = *reinterpret_cast<const float4v*>(row + col);
+    // Every split's part of four columns, requested before the first is added.
+    struct Parts
+    {
+        float4v v[kMaxGemmSplits];
+        float4v bias;
+    };
+    auto request = [&](uint32_t col) {
+        Parts p;
+        p.v[0] = *reinterpret_cast<const float4v*>(row + col);
         if (splits > 1)
         {
-            for (uint32_t z = 1; z < splits; ++z)
+#pragma unroll
+            for (uint32_t z = 1; z < kMaxGemmSplits; ++z)
             {
-                a += *reinterpret_cast<const float4v*>(row + z * stride + col);
+                if (z < splits)
+                {
+                    p.v[z] = *reinterpret_cast<const float4v*>(row + z * stride + col);
+                }
             }
-            a += *reinterpret_cast<const float4v*>(bias + col);
+            p.bias = *reinterpret_cast<const float4v*>(bias + col);
+        }
+        return p;
+    };
+    auto total = [&](const Parts& p) {
+        float4v a = p.v[0];
+        if (splits > 1)
+        {
+#pragma unroll
+            for (uint32_t z = 1; z < kMaxGemmSplits; ++z)
+            {
+                if (z < splits)
+                {
+                    a += p.v[z];
+                }
+            }
+            a += p.bias;
         }
         return a;
     };
@@ -419,8 +415,8 @@ __global__ __launch_bounds__(256) void RopeSplitAppendQuadKernel(const float* __
         const uint32_t head = unit / quads;
         const uint32_t j = (unit % quads) * 4;
         const float4v power = *reinterpret_cast<const float4v*>(ropePow + j);
-        const float4v s0 = value4(head * headDim + j);
-        const float4v s1 = value4(head * headDim + j + half);
+        const Parts p0 = request(head * headDim + j);
+        const Parts p1 = request(head * headDim + j + half);
         float c[4];
         float sn[4];
 #pragma unroll
@@ -429,6 +425,8 @@ __global__ __launch_bounds__(256) void RopeSplitAppendQuadKernel(const float* __
             const float theta = static_cast<float>(pos) * power[e];
             sincosf(theta, &sn[e], &c[e]);
         }
+        const float4v s0 = total(p0);
+        const float4v s1 = total(p1);
         float o0[4];
         float o1[4];
 #pragma unroll
@@ -459,389 +457,11 @@ __global__ __launch_bounds__(256) void RopeSplitAppendQuadKernel(const float* __
         const uint32_t channel = 4 * (unit - ropeUnits);  // within kvHeads * headDim
         const uint32_t g = channel / headDim;
         const uint64_t base = (static_cast<uint64_t>(g) * maxSeq + pos) * headDim + channel % headDim;
-        const float4v v = value4((heads + kvHeads) * headDim + channel);
+        const float4v v = total(request((heads + kvHeads) * headDim + channel));
         const ushort4v out = {FloatToHalfBits(v[0]), FloatToHalfBits(v[1]), FloatToHalfBits(v[2]),
                               FloatToHalfBits(v[3])};
         *reinterpret_cast<ushort4v*>(vcache + base) = out;
     }
-}
-
-// ------------------------------------------------------------------------------------------------
-// Split GEMM: out[m][n] = sum_k (ahi + alo)[m][k] * W[n][k]. Each wave owns a 64 (n) x 64 (m)
-// tile as 2 x 2 blocks of 32 x 32 accumulators; the weights are the matrix core's A operand
-// (rows n), the activation planes its B operand (columns m), so a lane ends with four
-// consecutive n of one m per accumulator group: 16-byte stores into row-major [m][n].
-// K advances 64 halves at a time through one LDS tile per operand (rows padded to 144 bytes, so
-// the 16-byte fragment reads of 8 consecutive rows touch distinct banks); the next tile's global
-// loads are in flight while the current one is multiplied.
-
-constexpr int kGemmBK = 64;
-constexpr int kGemmStride = kGemmBK + 8;
-
-/// out = acc + bias[n] + residual[m][n] (either may be null); virtual rows are the weight rows.
-/// With `partial` the grid splits K (blockIdx.z) and each split stores its raw sums to plane z of
-/// `partial` ([splits][rows][n]); bias and residual are then the consumer's to add.
-struct PlainEpi
-{
-    const uint16_t* w;
-    const float* bias;
-    const float* residual;
-    float* out;
-    uint32_t n, k;
-    float* partial = nullptr;
-
-    /// Weight rows u + r (r < 16 or 32, u a multiple of that): row u's index and address, uniform
-    /// across the workgroup (clamped to the last row); row u + r is r * k elements on.
-    __device__ uint32_t WFirst(uint32_t u) const { return u; }
-    __device__ uint32_t WCount() const { return n; }
-    __device__ const uint16_t* WRows(uint32_t u) const { return w + static_cast<uint64_t>(min(u, n - 1)) * k; }
-
-    template <int kNb>
-    __device__ void Finish(const floatx16 (&acc)[kNb][2], uint32_t n0, uint32_t m0, uint32_t rows) const
-    {
-        const uint32_t lane = threadIdx.x % kWave;
-        const uint32_t h = lane / 32;
-#pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
-        {
-            const uint32_t m = m0 + mb * 32 + lane % 32;
-            if (m >= rows)
-            {
-                continue;
-            }
-#pragma unroll
-            for (int nb = 0; nb < kNb; ++nb)
-            {
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-                {
-                    const uint32_t nn = n0 + nb * 32 + 8 * g + 4 * h;
-                    if (nn >= n)
-                    {
-                        continue;
-                    }
-                    float4 v = make_float4(acc[nb][mb][4 * g], acc[nb][mb][4 * g + 1], acc[nb][mb][4 * g + 2],
-                                           acc[nb][mb][4 * g + 3]);
-                    const uint64_t at = static_cast<uint64_t>(m) * n + nn;
-                    if (partial != nullptr)
-                    {
-                        *reinterpret_cast<float4*>(partial + static_cast<uint64_t>(blockIdx.z) * rows * n + at) = v;
-                        continue;
-                    }
-                    if (bias != nullptr)
-                    {
-                        const float4 b = *reinterpret_cast<const float4*>(bias + nn);
-                        v.x += b.x;
-                        v.y += b.y;
-                        v.z += b.z;
-                        v.w += b.w;
-                    }
-                    if (residual != nullptr)
-                    {
-                        const float4 r = *reinterpret_cast<const float4*>(residual + at);
-                        v.x = r.x + v.x;
-                        v.y = r.y + v.y;
-                        v.z = r.z + v.z;
-                        v.w = r.w + v.w;
-                    }
-                    *reinterpret_cast<float4*>(out + at) = v;
-                }
-            }
-        }
-    }
-};
-
-/// Gate and up interleaved per wave tile: virtual rows [64 t, 64 t + 32) are gate rows
-/// [32 t, 32 t + 32) and the next 32 the same up rows, so a lane holds g and u of the same
-/// (m, f) and writes silu(g) * u (swiglu.comp's op) as split planes.
-struct SwiGluEpi
-{
-    const uint16_t* gate;
-    const uint16_t* up;
-    uint16_t* hhi;
-    uint16_t* hlo;
-    uint32_t ffn, k;
-
-    /// Virtual rows u + r (r < 16 or 32, u a multiple of that) are gate or up rows f + r of one
-    /// matrix, f = (u / 64) * 32 + u % 32: uniform across the workgroup (the address clamped to
-    /// the last row).
-    __device__ uint32_t WFirst(uint32_t u) const { return (u / 64) * 32 + u % 32; }
-    __device__ uint32_t WCount() const { return ffn; }
-    __device__ const uint16_t* WRows(uint32_t u) const
-    {
-        return (u % 64 < 32 ? gate : up) + static_cast<uint64_t>(min(WFirst(u), ffn - 1)) * k;
-    }
-
-    /// Blocks 2p and 2p + 1 of a wave's kNb are the gate and up rows of the same 32 f.
-    template <int kNb>
-    __device__ void Finish(const floatx16 (&acc)[kNb][2], uint32_t n0, uint32_t m0, uint32_t rows) const
-    {
-        const uint32_t lane = threadIdx.x % kWave;
-        const uint32_t h = lane / 32;
-#pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
-        {
-            const uint32_t m = m0 + mb * 32 + lane % 32;
-            if (m >= rows)
-            {
-                continue;
-            }
-#pragma unroll
-            for (int p = 0; p < kNb / 2; ++p)
-            {
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-                {
-                    const uint32_t f = (n0 + 64 * p) / 2 + 8 * g + 4 * h;
-                    if (f >= ffn)
-                    {
-                        continue;
-                    }
-                    float a[4];
-#pragma unroll
-                    for (int t = 0; t < 4; ++t)
-                    {
-                        const float gv = acc[2 * p][mb][4 * g + t];
-                        a[t] = gv / (1.0f + expf(-gv)) * acc[2 * p + 1][mb][4 * g + t];
-                    }
-                    StoreSplit4(hhi, hlo, static_cast<uint64_t>(m) * ffn + f, a[0], a[1], a[2], a[3]);
-                }
-            }
-        }
-    }
-};
-
-/// The grid's z splits K into runs of kPerSplit (a multiple of kGemmBK) columns. A wave owns 64
-/// tokens and kNb blocks of 32 weight rows.
-///
-/// Workgroups are dispatched in linear order (x fastest), and those resident at once share what
-/// they read through L2 and the Infinity Cache. By default the grid's x walks the weight tiles,
-/// so consecutive workgroups share an activation tile. With `mFast` it walks the token tiles:
-/// consecutive workgroups share a weight slice, so a weight larger than the cache (the 7B
-/// gate+up's 272 MB) is read from HBM about once instead of once per round of resident token
-/// tiles, while the activation planes, the smaller operand, stay cached.
-template <int kWm, int kWn, typename Epi, int kNb = 2, int kStages = 1>
-__global__ __launch_bounds__(kWave * kWm * kWn, kNb == 4 || kStages == 2 ? 2 : 1) void GemmSplitKernel(const uint16_t* __restrict__ ahi,
-                                                                     const uint16_t* __restrict__ alo, Epi epi,
-                                                                     uint32_t rows, uint32_t k, uint32_t kPerSplit,
-                                                                     uint32_t mFast)
-{
-    constexpr int kThreads = kWave * kWm * kWn;
-    constexpr int kBM = 64 * kWm;
-    constexpr int kBN = 32 * kNb * kWn;
-    constexpr int kChunks = kGemmBK / 8;  // 16-byte chunks per tile row
-    constexpr int kALoads = 2 * kBM * kChunks / kThreads;
-    constexpr int kWLoads = kBN * kChunks / kThreads;
-    static_assert((2 * kBM * kChunks) % kThreads == 0 && (kBN * kChunks) % kThreads == 0, "tile loads");
-    __shared__ __attribute__((aligned(16))) uint16_t lds[(2 * kBM + kBN) * kGemmStride];
-
-    const uint32_t tid = threadIdx.x;
-    const uint32_t linear = blockIdx.x + gridDim.x * blockIdx.y;
-    const uint32_t m0 = (mFast != 0 ? linear % gridDim.y : blockIdx.y) * kBM;
-    const uint32_t n0 = (mFast != 0 ? linear / gridDim.y : blockIdx.x) * kBN;
-
-    // Each thread loads one 16-byte chunk (column `col`) of rows r0, r0 + kRowsPerPass, ... of the
-    // A planes and of the weight. A row group's address is uniform across the workgroup and the
-    // lane adds r0 * k + col, so the addresses cost one register (scalar base + vector offset)
-    // rather than a 64-bit pointer per load. A lane whose row is past the matrix reads its group's
-    // first row instead (in bounds; its products land in outputs that are not stored), so the
-    // loads need no branches.
-    constexpr uint32_t kRowsPerPass = kThreads / kChunks;
-    static_assert(kBM % kRowsPerPass == 0 && 32 % kRowsPerPass == 0, "row groups");
-    const uint32_t r0 = tid / kChunks;
-    const uint32_t col = (tid % kChunks) * 8;
-    const uint32_t laneOffset = r0 * k + col;
-    const uint32_t dst = r0 * kGemmStride + col;
-
-    const uint32_t kBegin = blockIdx.z * kPerSplit;
-    const uint32_t kEnd = min(k, kBegin + kPerSplit);
-    // kStages register buffers: the loads of tile t + kStages are issued as tile t's registers
-    // reach LDS, so each load has kStages tiles of matrix-core work to arrive in.
-    half8 aReg[kStages][kALoads];
-    half8 wReg[kStages][kWLoads];
-    auto load = [&](auto buf, uint32_t k0)
-    {
-        constexpr int b = decltype(buf)::value;
-        // A chunk past kEnd (only in a K tile that runs past it) reads the tile's first chunk of
-        // its row instead, and is zeroed below.
-        const bool past = k0 + kGemmBK > kEnd && k0 + col >= kEnd;
-        const uint32_t c = past ? 0u : col;
-        const uint32_t offset = past ? r0 * k : laneOffset;
-#pragma unroll
-        for (int i = 0; i < kALoads; ++i)
-        {
-            const uint32_t plane = i * kRowsPerPass / kBM;
-            const uint32_t row = m0 + i * kRowsPerPass % kBM;
-            const uint16_t* base = (plane == 0 ? ahi : alo) + static_cast<uint64_t>(min(row, rows - 1)) * k + k0;
-            aReg[b][i] = *reinterpret_cast<const half8*>(base + (row + r0 < rows ? offset : c));
-        }
-#pragma unroll
-        for (int i = 0; i < kWLoads; ++i)
-        {
-            const uint32_t u = n0 + i * kRowsPerPass;
-            const uint16_t* base = epi.WRows(u) + k0;
-            wReg[b][i] = *reinterpret_cast<const half8*>(base + (epi.WFirst(u) + r0 < epi.WCount() ? offset : c));
-        }
-        if (past)
-        {
-#pragma unroll
-            for (int i = 0; i < kALoads; ++i)
-            {
-                aReg[b][i] = half8{};
-            }
-#pragma unroll
-            for (int i = 0; i < kWLoads; ++i)
-            {
-                wReg[b][i] = half8{};
-            }
-        }
-    };
-
-    const uint32_t wave = tid / kWave;
-    const uint32_t lane = tid % kWave;
-    const uint32_t wm = wave / kWn;
-    const uint32_t wn = wave % kWn;
-    const uint32_t lrow = lane % 32;
-    const uint32_t lk = (lane / 32) * 8;
-    const uint16_t* wFrag = lds + (2 * kBM + wn * 32 * kNb + lrow) * kGemmStride + lk;
-    const uint16_t* hiFrag = lds + (wm * 64 + lrow) * kGemmStride + lk;
-    const uint16_t* loFrag = lds + (kBM + wm * 64 + lrow) * kGemmStride + lk;
-
-    floatx16 acc[kNb][2];
-#pragma unroll
-    for (int a = 0; a < kNb; ++a)
-    {
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-        {
-            acc[a][b] = floatx16{};
-        }
-    }
-
-    // One tile: its registers to LDS, the refill of the same registers kStages tiles ahead, then
-    // the tile's products.
-    auto tile = [&](auto buf, uint32_t k0)
-    {
-        constexpr int b = decltype(buf)::value;
-        __syncthreads();  // every wave is done with the previous tile
-#pragma unroll
-        for (int i = 0; i < kALoads; ++i)
-        {
-            // Plane p's row r sits at LDS row p * kBM + r, i.e. row i * kRowsPerPass + r0.
-            *reinterpret_cast<half8*>(lds + dst + i * kRowsPerPass * kGemmStride) = aReg[b][i];
-        }
-#pragma unroll
-        for (int i = 0; i < kWLoads; ++i)
-        {
-            *reinterpret_cast<half8*>(lds + dst + (2 * kBM + i * kRowsPerPass) * kGemmStride) = wReg[b][i];
-        }
-        __syncthreads();
-        if (k0 + kStages * kGemmBK < kEnd)
-        {
-            load(buf, k0 + kStages * kGemmBK);
-        }
-#pragma unroll
-        for (int s = 0; s < kGemmBK / 16; ++s)
-        {
-            half8 wf[kNb], xh[2], xl[2];
-#pragma unroll
-            for (int b = 0; b < kNb; ++b)
-            {
-                wf[b] = *reinterpret_cast<const half8*>(wFrag + b * 32 * kGemmStride + s * 16);
-            }
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-            {
-                xh[b] = *reinterpret_cast<const half8*>(hiFrag + b * 32 * kGemmStride + s * 16);
-                xl[b] = *reinterpret_cast<const half8*>(loFrag + b * 32 * kGemmStride + s * 16);
-            }
-            // The hi products of every block, then the lo products, so that independent
-            // matrix-core operations separate two that accumulate into the same block.
-#pragma unroll
-            for (int nb = 0; nb < kNb; ++nb)
-            {
-#pragma unroll
-                for (int mb = 0; mb < 2; ++mb)
-                {
-                    acc[nb][mb] = Mfma(wf[nb], xh[mb], acc[nb][mb]);
-                }
-            }
-#pragma unroll
-            for (int nb = 0; nb < kNb; ++nb)
-            {
-#pragma unroll
-                for (int mb = 0; mb < 2; ++mb)
-                {
-                    acc[nb][mb] = Mfma(wf[nb], xl[mb], acc[nb][mb]);
-                }
-            }
-        }
-    };
-
-    using First = std::integral_constant<int, 0>;
-    using Second = std::integral_constant<int, kStages - 1>;
-    load(First{}, kBegin);
-    if (kStages == 2 && kBegin + kGemmBK < kEnd)
-    {
-        load(Second{}, kBegin + kGemmBK);
-    }
-    for (uint32_t k0 = kBegin; k0 < kEnd; k0 += kStages * kGemmBK)
-    {
-        tile(First{}, k0);
-        if (kStages == 2 && k0 + kGemmBK < kEnd)
-        {
-            tile(Second{}, k0 + kGemmBK);
-        }
-    }
-    epi.Finish(acc, n0 + wn * 32 * kNb, m0 + wm * 64, rows);
-}
-
-/// 128 x 128 tiles when they, with the K splits, give two workgroups per CU, or unsplit fill at
-/// least seven eighths of that (448 of 512 on 256 CUs); 64-token tiles otherwise.
-bool BigTiles(uint32_t rows, uint32_t virtualRows, uint32_t splits = 1)
-{
-    const uint64_t tiles = static_cast<uint64_t>(CeilDiv(rows, 128)) * CeilDiv(virtualRows, 128);
-    return tiles * splits >= 512 || (splits == 1 && tiles * 8 >= 512 * 7);
-}
-
-/// 128-token x 256-row tiles (a wave 64 tokens x 128 rows, two workgroups per CU) when they give
-/// four workgroups per CU or more: an activation fragment read from LDS feeds twice the
-/// matrix-core work. With fewer tiles the last round's imbalance costs more than that gains,
-/// unless K splits make them one nearly full round (LaunchGemm).
-bool WideTiles(uint32_t rows, uint32_t virtualRows)
-{
-    return static_cast<uint64_t>(CeilDiv(rows, 128)) * CeilDiv(virtualRows, 256) >= 1024;
-}
-
-template <typename Epi>
-hipError_t LaunchGemm(hipStream_t s, const uint16_t* ahi, const uint16_t* alo, const Epi& epi, uint32_t rows,
-                      uint32_t virtualRows, uint32_t k, uint32_t splits = 1)
-{
-    if (rows == 0 || virtualRows == 0 || k == 0 || splits == 0)
-    {
-        return hipErrorInvalidValue;
-    }
-    const uint32_t kPerSplit = CeilDiv(CeilDiv(k, kGemmBK), splits) * kGemmBK;
-    // Token tiles fastest where the weight outweighs the activation planes and K is whole (the
-    // gate+up GEMMs: 7B 1200 -> 1087 us; the K-split q|k|v and o_proj measured slower so).
-    const uint32_t mFast = splits == 1 && static_cast<uint64_t>(virtualRows) * 2 > static_cast<uint64_t>(rows) * 4;
-    const uint64_t wideSplits = static_cast<uint64_t>(CeilDiv(rows, 128)) * CeilDiv(virtualRows, 256) * splits;
-    if (WideTiles(rows, virtualRows) || (splits > 1 && wideSplits * 8 >= 512 * 7 && wideSplits <= 512))
-    {
-        hipLaunchKernelGGL((GemmSplitKernel<2, 2, Epi, 4, 1>), dim3(CeilDiv(virtualRows, 256), CeilDiv(rows, 128), splits),
-                           dim3(256), 0, s, ahi, alo, epi, rows, k, kPerSplit, mFast);
-    }
-    else if (BigTiles(rows, virtualRows, splits))
-    {
-        hipLaunchKernelGGL((GemmSplitKernel<2, 2, Epi, 2, 2>), dim3(CeilDiv(virtualRows, 128), CeilDiv(rows, 128), splits),
-                           dim3(256), 0, s, ahi, alo, epi, rows, k, kPerSplit, mFast);
-    }
-    else
-    {
-        hipLaunchKernelGGL((GemmSplitKernel<1, 2, Epi, 2, 2>), dim3(CeilDiv(virtualRows, 128), CeilDiv(rows, 64), splits),
-                           dim3(128), 0, s, ahi, alo, epi, rows, k, kPerSplit, mFast);
-    }
-    return hipGetLastError();
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1231,76 +851,6 @@ hipError_t LaunchSplitF32(hipStream_t s, const float* x, uint64_t count, uint16_
     const uint32_t blocks = static_cast<uint32_t>(quads / 256 + 1 < 4096 ? quads / 256 + 1 : 4096);
     hipLaunchKernelGGL(SplitF32Kernel, dim3(blocks), dim3(256), 0, s, x, quads, hi, lo);
     return hipGetLastError();
-}
-
-uint32_t GemmSplits(uint32_t rows, uint32_t n, uint32_t k)
-{
-    if (rows == 0 || n == 0)
-    {
-        return 1;
-    }
-    const uint64_t bigTiles = static_cast<uint64_t>(CeilDiv(rows, 128)) * CeilDiv(n, 128);
-    const bool halves = CeilDiv(k, kGemmBK) >= 8;
-    // 128 x 128 tiles alone fill two workgroups per CU: K halves when under four per CU.
-    if (bigTiles >= 512)
-    {
-        return bigTiles < 1024 && halves ? 2 : 1;
-    }
-    // 128 x 256 tiles over two K halves that fill seven eighths to all of one round (7B o_proj
-    // and down, 448 workgroups): the wide tiles' matrix-core work per LDS read outweighs the
-    // partial planes the next norm sums (o_proj + down 727 -> 614 us, the norms 18 -> 37 us).
-    const uint64_t wideHalves = static_cast<uint64_t>(CeilDiv(rows, 128)) * CeilDiv(n, 256) * 2;
-    if (halves && wideHalves * 8 >= 512 * 7 && wideHalves <= 512)
-    {
-        return 2;
-    }
-    // Otherwise at least seven eighths of one round of 128 x 128 tiles: unsplit, with no partial
-    // planes for the next norm to sum.
-    if (bigTiles * 8 >= 512 * 7)
-    {
-        return 1;
-    }
-    // 128 x 128 tiles over two K halves, where that grid fills two workgroups per CU.
-    if (bigTiles * 2 >= 512 && halves)
-    {
-        return 2;
-    }
-    // 64-token tiles: waves of the unsplit grid (64 x 64 outputs each); short of ~1024 (a wave
-    // per SIMD), K is split so the grid reaches it, keeping at least two K tiles per split.
-    const uint64_t waves = static_cast<uint64_t>(CeilDiv(rows, 64)) * CeilDiv(n, 128) * 2;
-    const uint32_t tiles = CeilDiv(k, kGemmBK);
-    uint32_t splits = static_cast<uint32_t>(std::min<uint64_t>(kMaxGemmSplits, CeilDiv(1024, waves)));
-    while (splits > 1 && tiles / splits < 2)
-    {
-        --splits;
-    }
-    return std::max(splits, 1u);
-}
-
-hipError_t LaunchGemmSplit(hipStream_t s, const uint16_t* ahi, const uint16_t* alo, const uint16_t* w,
-                           const float* bias, const float* residual, float* out, uint32_t rows, uint32_t n,
-                           uint32_t k, float* partial, uint32_t splits)
-{
-    if (n % 4 != 0 || k % 8 != 0 || splits == 0 || splits > kMaxGemmSplits || (splits > 1 && partial == nullptr))
-    {
-        return hipErrorInvalidValue;
-    }
-    PlainEpi epi{w, bias, residual, out, n, k};
-    epi.partial = splits > 1 ? partial : nullptr;
-    return LaunchGemm(s, ahi, alo, epi, rows, n, k, splits);
-}
-
-hipError_t LaunchGemmSwiGlu(hipStream_t s, const uint16_t* ahi, const uint16_t* alo, const uint16_t* wgate,
-                            const uint16_t* wup, uint16_t* hhi, uint16_t* hlo, uint32_t rows, uint32_t ffn,
-                            uint32_t k)
-{
-    if (ffn % 4 != 0 || k % 8 != 0)
-    {
-        return hipErrorInvalidValue;
-    }
-    // Two virtual rows (gate, up) per output, in whole 32-row blocks.
-    const uint32_t virtualRows = 2 * CeilDiv(ffn, 32) * 32;
-    return LaunchGemm(s, ahi, alo, SwiGluEpi{wgate, wup, hhi, hlo, ffn, k}, rows, virtualRows, k);
 }
 
 hipError_t LaunchRopeSplitAppend(hipStream_t s, const float* qkv, uint32_t rows, int32_t pos0, uint32_t heads,

@@ -27,8 +27,18 @@ hipError_t LaunchRmsNormSplit(hipStream_t s, const float* x, const float* w, uin
 /// hi/lo planes of a plain f32 matrix (no norm): count values, count % 4 == 0.
 hipError_t LaunchSplitF32(hipStream_t s, const float* x, uint64_t count, uint16_t* hi, uint16_t* lo);
 
-/// Most K splits of a prefill GEMM.
-constexpr uint32_t kMaxGemmSplits = 4;
+/// Most K splits of a prefill GEMM: eight while the partial planes of that many stay small.
+constexpr uint32_t kMaxGemmSplits = 8;
+constexpr uint32_t kFewRows = 512;
+inline uint32_t MaxGemmSplits(uint32_t rows) { return rows <= kFewRows ? kMaxGemmSplits : kMaxGemmSplits / 2; }
+
+/// Floats of the partial planes of any GEMM of up to `rows` rows and `n` columns.
+inline size_t GemmPartialFloats(uint32_t rows, uint32_t n)
+{
+    const size_t few = static_cast<size_t>(kMaxGemmSplits) * (rows < kFewRows ? rows : kFewRows);
+    const size_t many = static_cast<size_t>(kMaxGemmSplits / 2) * rows;
+    return (few > many ? few : many) * n;
+}
 constexpr uint32_t kAttnMaxChunks = 8;    // key chunks a split prefill-attention query tile takes at most
 constexpr uint32_t kAttnMaxItems = 512;   // work items of one split attention launch (64 tiles x 8)
 
@@ -38,8 +48,8 @@ inline size_t PrefillAttentionWorkspaceFloats(uint32_t rows, uint32_t heads, uin
     return static_cast<size_t>(kAttnMaxChunks) * rows * heads * (headDim + 2);
 }
 
-/// K splits for a GEMM of this shape: more than one when its output tiles alone leave most SIMDs
-/// without a wave (the 0.5B shape's q|k|v, o_proj and down at 2048 rows).
+/// K splits for a GEMM of this shape: more than one when its output tiles alone leave CUs idle and
+/// the partial planes cost less than that (at most MaxGemmSplits(rows)).
 uint32_t GemmSplits(uint32_t rows, uint32_t n, uint32_t k);
 
 /// out[m][n] = sum_k (ahi + alo)[m][k] * w[n][k] + bias[n] (bias may be null) + residual[m][n]

@@ -1,0 +1,646 @@
+// Split-f16 GEMMs of the batched prefill: out[m][n] = sum_k (ahi + alo)[m][k] * W[n][k] on
+// v_mfma_f32_32x32x16_f16, with fused epilogues.
+//
+// The weights are the matrix core's A operand (rows n), the activation planes its B operand
+// (columns m), so a lane ends with four consecutive n of one m per accumulator group: 16-byte
+// stores into row-major [m][n]. Each weight fragment meets the hi and the lo plane.
+#include <algorithm>
+#include <cmath>
+#include <limits>
+
+#include "prefill.hpp"
+#include "prefill_core.hpp"
+
+namespace muyo
+{
+namespace
+{
+/// K is split on multiples of this many columns (the widest K slab of a tile shape).
+constexpr uint32_t kGemmSplitUnit = 128;
+
+/// out = acc + bias[n] + residual[m][n] (either may be null); virtual rows are the weight rows.
+/// With `partial` each K split z stores its raw sums to plane z of `partial` ([splits][rows][n]);
+/// bias and residual are then the consumer's to add.
+struct PlainEpi
+{
+    const uint16_t* w;
+    const float* bias;
+    const float* residual;
+    float* out;
+    uint32_t n, k;
+    float* partial = nullptr;
+
+    /// LDS row that holds virtual row v of a 32-row block.
+    __device__ static uint32_t LdsRow(uint32_t v) { return v; }
+    /// The matrix row in LDS row u (uniform; clamped to the last row), and whether u + r exists.
+    __device__ const uint16_t* Row(uint32_t u) const { return w + static_cast<uint64_t>(min(u, n - 1)) * k; }
+    __device__ bool Live(uint32_t u, uint32_t r) const { return u + r < n; }
+
+    template <int kNb, int kMb>
+    __device__ void Finish(const floatx16 (&acc)[kNb][kMb], uint32_t n0, uint32_t m0, uint32_t rows, uint32_t z) const
+    {
+        const uint32_t lane = threadIdx.x % kWave;
+        const uint32_t h = lane / 32;
+#pragma unroll
+        for (int mb = 0; mb < kMb; ++mb)
+        {
+            const uint32_t m = m0 + mb * 32 + lane % 32;
+            if (m >= rows)
+            {
+                continue;
+            }
+#pragma unroll
+            for (int nb = 0; nb < kNb; ++nb)
+            {
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                {
+                    const uint32_t nn = n0 + nb * 32 + 8 * g + 4 * h;
+                    if (nn >= n)
+                    {
+                        continue;
+                    }
+                    float4 v = make_float4(acc[nb][mb][4 * g], acc[nb][mb][4 * g + 1], acc[nb][mb][4 * g + 2],
+                                           acc[nb][mb][4 * g + 3]);
+                    const uint64_t at = static_cast<uint64_t>(m) * n + nn;
+                    if (partial != nullptr)
+                    {
+                        *reinterpret_cast<float4*>(partial + static_cast<uint64_t>(z) * rows * n + at) = v;
+                        continue;
+                    }
+                    if (bias != nullptr)
+                    {
+                        const float4 b = *reinterpret_cast<const float4*>(bias + nn);
+                        v.x += b.x;
+                        v.y += b.y;
+                        v.z += b.z;
+                        v.w += b.w;
+                    }
+                    if (residual != nullptr)
+                    {
+                        const float4 r = *reinterpret_cast<const float4*>(residual + at);
+                        v.x = r.x + v.x;
+                        v.y = r.y + v.y;
+                        v.z = r.z + v.z;
+                        v.w = r.w + v.w;
+                    }
+                    *reinterpret_cast<float4*>(out + at) = v;
+                }
+            }
+        }
+    }
+};
+
+/// Gate and up interleaved eight rows at a time, so that any 32-row block is complete: virtual
+/// rows 16 t + j are gate row 8 t + j for j < 8 and up row 8 t + j - 8 for the other eight. A lane
+/// then holds g (accumulator groups 0 and 2) and u (1 and 3) of the same (m, f) and writes
+/// silu(g) * u (swiglu.comp's op) as split planes. In LDS a block's 16 gate rows come first, so
+/// that the rows one load instruction brings are neighbours in one matrix.
+struct SwiGluEpi
+{
+    const uint16_t* gate;
+    const uint16_t* up;
+    uint16_t* hhi;
+    uint16_t* hlo;
+    uint32_t ffn, k;
+
+    __device__ static uint32_t LdsRow(uint32_t v) { return (v & 8u) * 2 + (v >> 4) * 8 + (v & 7u); }
+    __device__ static uint32_t First(uint32_t u) { return u / 32 * 16 + u % 16; }
+    __device__ const uint16_t* Row(uint32_t u) const
+    {
+        return (u % 32 < 16 ? gate : up) + static_cast<uint64_t>(min(First(u), ffn - 1)) * k;
+    }
+    __device__ bool Live(uint32_t u, uint32_t r) const { return First(u) + r < ffn; }
+
+    template <int kNb, int kMb>
+    __device__ void Finish(const floatx16 (&acc)[kNb][kMb], uint32_t n0, uint32_t m0, uint32_t rows, uint32_t) const
+    {
+        const uint32_t lane = threadIdx.x % kWave;
+        const uint32_t h = lane / 32;
+#pragma unroll
+        for (int mb = 0; mb < kMb; ++mb)
+        {
+            const uint32_t m = m0 + mb * 32 + lane % 32;
+            if (m >= rows)
+            {
+                continue;
+            }
+#pragma unroll
+            for (int nb = 0; nb < kNb; ++nb)
+            {
+#pragma unroll
+                for (int g = 0; g < 4; g += 2)
+                {
+                    const uint32_t f = (n0 + nb * 32) / 2 + 4 * g + 4 * h;
+                    if (f >= ffn)
+                    {
+                        continue;
+                    }
+                    float a[4];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                    {
+                        const float gv = acc[nb][mb][4 * g + t];
+                        a[t] = gv / (1.0f + expf(-gv)) * acc[nb][mb][4 * g + 4 + t];
+                    }
+                    StoreSplit4(hhi, hlo, static_cast<uint64_t>(m) * ffn + f, a[0], a[1], a[2], a[3]);
+                }
+            }
+        }
+    }
+};
+
+/// Waits until at most kLeft of this wave's loads are in flight and its LDS reads are done, then
+/// meets the other waves.
+template <int kLeft>
+__device__ __forceinline__ void WaitAndMeet()
+{
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kLeft) : "memory");
+}
+
+/// A tile of kBm tokens x kBn weight rows by kWm x kWn x kWk waves: a wave owns kMb x kNb blocks
+/// of 32 x 32 outputs, and with kWk > 1 that many waves own the same blocks and every kWk-th step
+/// of 16 columns, their sums meeting in LDS at the end.
+///
+/// K advances kBk columns at a time through kStages LDS buffers. The loads go from memory to LDS
+/// without passing through registers (global_load_lds_dwordx4: a wave's 64 x 16 bytes land in 1 KB
+/// of LDS in lane order), up to kStages - 1 slabs ahead, and a slab costs one barrier: past it,
+/// every wave's part of the slab has arrived and every wave is done with the buffer that the next
+/// loads overwrite. Rows are not padded (the load writes 1 KB at a stretch), so each row's 16-byte
+/// chunks are permuted by the row number instead, on the global side of the load; the fragment
+/// reads of eight consecutive rows then touch every bank once.
+///
+/// The compiler does not see these loads: it neither counts them nor orders LDS reads after
+/// them. WaitAndMeet counts them (a wave's loads complete in order, kLoads a slab).
+///
+/// What bounds it. With random data the matrix cores alone sustain 1.67 PFLOP/s on this part (its
+/// power limit; 2.3 with zeros), and 1.5 with an LDS fragment read for every two operations. Loads
+/// from L2 run at 34 TB/s but anything past it at 7, so a tile order that lets every XCD fetch
+/// every weight row is bound by that: workgroups are dealt to the XCDs round-robin, and XCD x
+/// takes the x-th eighth of the tiles instead (GemmOrder), 3.3 MB of each XCD's own rather than
+/// all 17 MB of the 0.5B gate+up weight. A single wave per SIMD leaves the matrix cores idle
+/// between a barrier and its first fragments: the shapes have two (or two workgroups per CU) where
+/// LDS allows.
+/// Measured, before (a register-staged kernel, one LDS buffer) and now, us: 0.5B gate+up
+/// 301 rows 29.5 / 18.4, 613 rows 36.7 / 29.9; down 301 rows 82 / 24; 613 rows over K splits
+/// 34 / 22.5; q|k|v 613 rows 12.5 / 8.7; 7B gate+up 45 rows 91 / 55, 2048 rows 999 / 936; down
+/// 45 rows 78 / 36, 2048 rows 494 / 467.
+template <int kWm, int kWn, int kWk, int kMb, int kNb, int kStages, int kBk, int kPerCu>
+struct GemmTile
+{
+    static constexpr int kWaves = kWm * kWn * kWk;
+    static constexpr int kThreads = kWave * kWaves;
+    static constexpr int kBm = 32 * kMb * kWm;
+    static constexpr int kBn = 32 * kNb * kWn;
+    static constexpr int kRows = 2 * kBm + kBn;           // LDS rows of a slab: hi, lo, weights
+    static constexpr int kRowBytes = 2 * kBk;
+    static constexpr int kChunks = kBk / 8;               // 16-byte chunks per row
+    static constexpr int kRowsPerLoad = kWave / kChunks;  // rows one load instruction brings
+    static constexpr int kGroups = kRows / kRowsPerLoad;
+    static constexpr int kLoads = (kGroups + kWaves - 1) / kWaves;  // per wave and slab
+    static constexpr int kStageBytes = kRows * kRowBytes;
+    static constexpr int kSteps = kBk / 16 / kWk;         // per wave and slab
+    static constexpr int kMinWaves = (kWaves * kPerCu + 3) / 4;  // per SIMD
+    static constexpr int kMaxBlocks = kPerCu;             // workgroups a CU holds (by LDS)
+    static constexpr bool kLowSums = kMb * kNb <= 4;      // two sums per block
+    static constexpr int kSumFloats = 1024 * kNb * kMb;   // a wave's tile
+    static_assert(kRows % kRowsPerLoad == 0 && kBm % kRowsPerLoad == 0 && 16 % kRowsPerLoad == 0, "row groups");
+    static_assert(kBk % (16 * kWk) == 0 && kGemmSplitUnit % kBk == 0, "steps");
+    static_assert(kStages >= 2 && kStages <= 5 && kStages * kStageBytes * kPerCu <= 160 * 1024, "LDS");
+    static_assert((kWk - 1) * kWm * kWn * kSumFloats * 4 <= kStages * kStageBytes, "LDS of the K sums");
+};
+
+/// This workgroup's tile and K split. Workgroups are dealt to the 8 XCDs round-robin by id; with
+/// the renumbering XCD x runs a contiguous run of the sequence (split, then weight tiles, then
+/// token tiles fastest, or the last two swapped), so its L2 holds its own share of the slower
+/// dimension. Which dimension is the slower one: the larger operand's, read once over the chip
+/// while the other is read by every XCD. (The results do not depend on where a workgroup runs.)
+struct GemmOrder
+{
+    uint32_t mTiles, nTiles;
+    bool mFast;
+
+    __device__ void Tile(uint32_t& mt, uint32_t& nt, uint32_t& z) const
+    {
+        const uint32_t xcd = blockIdx.x % 8;
+        const uint32_t id = xcd * (gridDim.x / 8) + min(xcd, gridDim.x % 8) + blockIdx.x / 8;
+        const uint32_t plane = mTiles * nTiles;
+        z = id / plane;
+        const uint32_t t = id % plane;
+        mt = mFast ? t % mTiles : t / nTiles;
+        nt = mFast ? t / mTiles : t % nTiles;
+    }
+};
+
+template <typename T, int kWm, int kWn, int kWk, int kMb, int kNb, int kStages, int kBk, typename Epi>
+__global__ __launch_bounds__(T::kThreads, T::kMinWaves) void GemmSplitKernel(const uint16_t* __restrict__ ahi,
+                                                                             const uint16_t* __restrict__ alo, Epi epi,
+                                                                             uint32_t rows, uint32_t k,
+                                                                             uint32_t kPerSplit, GemmOrder order)
+{
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[kStages * T::kStageBytes];
+    constexpr uint32_t kAGroups = 2 * T::kBm / T::kRowsPerLoad;
+
+    const uint32_t lane = threadIdx.x % kWave;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    uint32_t mt, nt, z;
+    order.Tile(mt, nt, z);
+    const uint32_t m0 = mt * T::kBm;
+    const uint32_t n0 = nt * T::kBn;
+    const uint32_t kBegin = z * kPerSplit;
+    const uint32_t kEnd = min(k, kBegin + kPerSplit);
+    const uint32_t slabs = kBegin < kEnd ? (kEnd - kBegin + kBk - 1) / kBk : 0;
+
+    // Load i of a wave brings LDS rows [g * kRowsPerLoad, ...) of a slab. The address is a row
+    // group's, uniform across the wave, plus the lane's offset. A lane whose row lies past the
+    // matrix reads the group's first row (clamped to the last) instead, and one whose chunk lies
+    // past kEnd the row's first chunk of the slab: in bounds, and either not stored or zeroed
+    // below. A wave with fewer groups than kLoads brings its last one again, so that the counts
+    // of WaitAndMeet hold for every wave.
+    const uint32_t groupRow = lane / T::kChunks;
+    const uint32_t ldsBase =
+        static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)lds));
+    auto load = [&](uint32_t stage, uint32_t k0, int i)
+    {
+        const uint32_t g = min(wave + i * T::kWaves, static_cast<uint32_t>(T::kGroups) - 1);
+        const uint32_t r = g * T::kRowsPerLoad;
+        const uint32_t row = r + groupRow;
+        const uint32_t chunk = (lane % T::kChunks) ^ (kBk == 32 ? (row >> 1) & 3u : row & 7u);
+        const uint32_t first = (k0 + (k0 + chunk * 8 < kEnd ? chunk * 8 : 0u)) * 2;
+        const uint16_t* base;
+        bool live;
+        if (g < kAGroups)
+        {
+            const bool lo = r >= T::kBm;
+            const uint32_t m = m0 + (lo ? r - T::kBm : r);
+            base = (lo ? alo : ahi) + static_cast<uint64_t>(min(m, rows - 1)) * k;
+            live = m + groupRow < rows;
+        }
+        else
+        {
+            const uint32_t u = n0 + r - 2 * T::kBm;
+            base = epi.Row(u);
+            live = epi.Live(u, groupRow);
+        }
+        const uint32_t offset = live ? first + groupRow * k * 2 : first;
+        const uint32_t to = ldsBase + stage * T::kStageBytes + g * 1024;
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(offset), "s"(base));
+    };
+
+    const uint32_t kg = wave / (kWm * kWn);
+    const uint32_t wm = wave / kWn % kWm;
+    const uint32_t wn = wave % kWn;
+    const uint32_t h = lane / 32;
+    const uint32_t aRow = lane % 32;
+    const uint32_t wRow = Epi::LdsRow(lane % 32);
+    const uint32_t aSwizzle = kBk == 32 ? (aRow >> 1) & 3u : aRow & 7u;
+    const uint32_t wSwizzle = kBk == 32 ? (wRow >> 1) & 3u : wRow & 7u;
+
+    // The lo products (2^-11 of the hi products) have sums of their own where the registers allow:
+    // half as many roundings at the size of the result.
+    floatx16 acc[kNb][kMb];
+    floatx16 low[T::kLowSums ? kNb : 1][T::kLowSums ? kMb : 1];
+#pragma unroll
+    for (int a = 0; a < kNb; ++a)
+    {
+#pragma unroll
+        for (int b = 0; b < kMb; ++b)
+        {
+            acc[a][b] = floatx16{};
+            if constexpr (T::kLowSums)
+            {
+                low[a][b] = floatx16{};
+            }
+        }
+    }
+#pragma unroll
+    for (uint32_t s = 0; s < kStages - 1; ++s)
+    {
+        if (s < slabs)
+        {
+#pragma unroll
+            for (int i = 0; i < T::kLoads; ++i)
+            {
+                load(s, kBegin + s * kBk, i);
+            }
+        }
+    }
+    uint32_t stage = 0;
+    for (uint32_t s = 0; s < slabs; ++s)
+    {
+        // The slabs after this one that are already requested stay in flight.
+        const uint32_t ahead = min(static_cast<uint32_t>(kStages - 2), slabs - 1 - s);
+        if (kStages <= 2 || ahead == 0)
+        {
+            WaitAndMeet<0>();
+        }
+        else if (kStages == 3 || ahead == 1)
+        {
+            WaitAndMeet<T::kLoads>();
+        }
+        else if (kStages == 4 || ahead == 2)
+        {
+            WaitAndMeet<2 * T::kLoads>();
+        }
+        else
+        {
+            WaitAndMeet<3 * T::kLoads>();
+        }
+        const bool more = s + kStages - 1 < slabs;
+        const uint32_t freed = stage == 0 ? kStages - 1 : stage - 1;
+        const uint8_t* tile = lds + stage * T::kStageBytes;
+#pragma unroll
+        for (int q = 0; q < T::kSteps; ++q)
+        {
+            const uint32_t step = q * kWk + kg;
+            const uint32_t aAt = ((step * 2 + h) ^ aSwizzle) * 16 + aRow * T::kRowBytes;
+            const uint32_t wAt = ((step * 2 + h) ^ wSwizzle) * 16 + wRow * T::kRowBytes;
+            half8 wf[kNb], xh[kMb], xl[kMb];
+#pragma unroll
+            for (int b = 0; b < kNb; ++b)
+            {
+                wf[b] = *reinterpret_cast<const half8*>(tile + (2 * T::kBm + (wn * kNb + b) * 32) * T::kRowBytes + wAt);
+            }
+#pragma unroll
+            for (int b = 0; b < kMb; ++b)
+            {
+                const uint8_t* x = tile + (wm * kMb + b) * 32 * T::kRowBytes + aAt;
+                xh[b] = *reinterpret_cast<const half8*>(x);
+                xl[b] = *reinterpret_cast<const half8*>(x + T::kBm * T::kRowBytes);
+            }
+            if (s + 1 == slabs && kBegin + s * kBk + step * 16 + 8 * h >= kEnd)
+            {
+#pragma unroll
+                for (int b = 0; b < kNb; ++b)
+                {
+                    wf[b] = half8{};
+                }
+#pragma unroll
+                for (int b = 0; b < kMb; ++b)
+                {
+                    xh[b] = half8{};
+                    xl[b] = half8{};
+                }
+            }
+            // The hi products of every block, then the lo products, so that independent
+            // matrix-core operations separate two that accumulate into the same block.
+#pragma unroll
+            for (int a = 0; a < kNb; ++a)
+            {
+#pragma unroll
+                for (int b = 0; b < kMb; ++b)
+                {
+                    acc[a][b] = Mfma(wf[a], xh[b], acc[a][b]);
+                }
+            }
+            // A step's share of the loads, spread over the slab: issued at once, they would hold
+            // the wave at the address unit before its first product.
+            if (more)
+            {
+#pragma unroll
+                for (int i = q * T::kLoads / T::kSteps; i < (q + 1) * T::kLoads / T::kSteps; ++i)
+                {
+                    load(freed, kBegin + (s + kStages - 1) * kBk, i);
+                }
+            }
+#pragma unroll
+            for (int a = 0; a < kNb; ++a)
+            {
+#pragma unroll
+                for (int b = 0; b < kMb; ++b)
+                {
+                    if constexpr (T::kLowSums)
+                    {
+                        low[a][b] = Mfma(wf[a], xl[b], low[a][b]);
+                    }
+                    else
+                    {
+                        acc[a][b] = Mfma(wf[a], xl[b], acc[a][b]);
+                    }
+                }
+            }
+        }
+        stage = stage + 1 == kStages ? 0 : stage + 1;
+    }
+    if constexpr (T::kLowSums)
+    {
+#pragma unroll
+        for (int a = 0; a < kNb; ++a)
+        {
+#pragma unroll
+            for (int b = 0; b < kMb; ++b)
+            {
+                acc[a][b] += low[a][b];
+            }
+        }
+    }
+    if constexpr (kWk > 1)
+    {
+        // K groups 1.. leave their tiles in LDS (done with as slabs), group 0 adds them in order.
+        __syncthreads();
+        float* sums = reinterpret_cast<float*>(lds);
+        if (kg > 0)
+        {
+            float* to = sums + (wave - kWm * kWn) * T::kSumFloats + lane * 4;
+#pragma unroll
+            for (int a = 0; a < kNb; ++a)
+            {
+#pragma unroll
+                for (int b = 0; b < kMb; ++b)
+                {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                    {
+                        *reinterpret_cast<float4*>(to + ((a * kMb + b) * 4 + q) * 256) =
+                            make_float4(acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2],
+                                        acc[a][b][4 * q + 3]);
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        if (kg > 0)
+        {
+            return;
+        }
+#pragma unroll 1
+        for (int other = 0; other < kWk - 1; ++other)
+        {
+            const float* from = sums + (other * kWm * kWn + wave) * T::kSumFloats + lane * 4;
+#pragma unroll
+            for (int a = 0; a < kNb; ++a)
+            {
+#pragma unroll
+                for (int b = 0; b < kMb; ++b)
+                {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                    {
+                        const float4 v = *reinterpret_cast<const float4*>(from + ((a * kMb + b) * 4 + q) * 256);
+                        acc[a][b][4 * q] += v.x;
+                        acc[a][b][4 * q + 1] += v.y;
+                        acc[a][b][4 * q + 2] += v.z;
+                        acc[a][b][4 * q + 3] += v.w;
+                    }
+                }
+            }
+        }
+    }
+    epi.Finish(acc, n0 + wn * 32 * kNb, m0 + wm * 32 * kMb, rows, z);
+}
+
+/// The tile shapes, X(index, waves m, n, k, blocks m, n, LDS stages, K slab, workgroups per CU).
+/// Seven of eighteen that were measured over the prefill's GEMMs (both models' four matrices, 7 to
+/// 2048 rows, every K split): with these seven the best choice per GEMM is within 1 % of the best
+/// of all eighteen on average.
+#define MUYO_GEMM_TILES(X)         \
+    X(0, 4, 2, 1, 2, 4, 3, 32, 1)  \
+    X(1, 2, 2, 2, 2, 3, 2, 64, 1)  \
+    X(2, 2, 4, 1, 1, 2, 3, 64, 1)  \
+    X(3, 2, 2, 2, 1, 3, 4, 64, 1)  \
+    X(4, 1, 2, 2, 1, 2, 3, 64, 2)  \
+    X(5, 1, 2, 4, 1, 2, 3, 128, 1) \
+    X(6, 1, 1, 4, 1, 2, 3, 128, 1)
+
+/// What the choice of a shape needs to know. slabUs is the time of 64 columns of K with the CUs
+/// busy, tileUs what a round of tiles costs besides (first loads, epilogue), both fitted to those
+/// measurements.
+struct GemmTileCost
+{
+    uint32_t bm, bn, bk, stages, perCu;
+    double slabUs, tileUs;
+};
+
+constexpr GemmTileCost kGemmTiles[] = {
+    {256, 256, 32, 3, 1, 2.70, 9.8}, {128, 192, 64, 2, 1, 1.57, 3.5}, {64, 256, 64, 3, 1, 0.875, 2.4},
+    {64, 192, 64, 4, 1, 0.69, 3.4},  {32, 128, 64, 3, 2, 0.67, 1.4},  {32, 128, 128, 3, 1, 0.354, 2.5},
+    {32, 64, 128, 3, 1, 0.287, 2.4},
+};
+constexpr int kGemmTileCount = sizeof(kGemmTiles) / sizeof(kGemmTiles[0]);
+constexpr uint32_t kCus = 256;
+
+/// Columns of K per split.
+uint32_t ColumnsPerSplit(uint32_t k, uint32_t splits)
+{
+    return CeilDiv(CeilDiv(k, kGemmSplitUnit), splits) * kGemmSplitUnit;
+}
+
+/// Estimated us of a launch of `tile` over `splits` K splits, with the partial planes' cost at
+/// their consumer: the rounds of resident workgroups times their slabs, or the time the weights
+/// take to arrive with the bytes each round keeps in flight (2 us each, at most 6 TB/s), whichever
+/// is longer. It ranks the shapes: over the measured GEMMs (88 with their own choice of splits, 88
+/// unsplit) the chosen one was 1.3 % slower than the fastest on average, 20 % at most.
+double GemmCost(const GemmTileCost& tile, uint32_t rows, uint32_t n, uint32_t k, uint32_t splits)
+{
+    const double tiles = static_cast<double>(CeilDiv(rows, tile.bm)) * CeilDiv(n, tile.bn) * splits;
+    const double slots = static_cast<double>(kCus) * tile.perCu;
+    const double fullRounds = std::floor(tiles / slots);
+    const double last = tiles - fullRounds * slots;
+    const double rounds = fullRounds + (last > 0.0 ? 1.0 : 0.0);
+    const double slabs = std::min(CeilDiv(k, 64), ColumnsPerSplit(k, splits) / 64);
+    const double alone = tile.perCu > 1 && tiles <= kCus ? 0.6 : 1.0;  // a CU's workgroups slow one another
+    const double tileBytes = 2.0 * n * k / tiles;
+    const double inFlight = static_cast<double>(tile.stages - 1) * tile.bn * tile.bk * 2;
+    auto arrive = [&](double count) { return count * tileBytes / std::min(6.0e6, count * inFlight / 2.0); };
+    const double weights = fullRounds * arrive(slots) + (last > 0.0 ? arrive(last) : 0.0);
+    const double partial = splits > 1 ? 1.0 + 12.0 * splits * rows * n / 4.0e6 : 0.0;
+    return 2.0 + std::max(rounds * (slabs * tile.slabUs * alone + tile.tileUs), weights + tile.tileUs) + partial;
+}
+
+template <typename Epi>
+hipError_t LaunchGemm(hipStream_t s, const uint16_t* ahi, const uint16_t* alo, const Epi& epi, uint32_t rows,
+                      uint32_t virtualRows, uint32_t k, uint32_t splits = 1)
+{
+    if (rows == 0 || virtualRows == 0 || k == 0 || splits == 0)
+    {
+        return hipErrorInvalidValue;
+    }
+    int best = 0;
+    for (int i = 1; i < kGemmTileCount; ++i)
+    {
+        if (GemmCost(kGemmTiles[i], rows, virtualRows, k, splits) < GemmCost(kGemmTiles[best], rows, virtualRows, k, splits))
+        {
+            best = i;
+        }
+    }
+    // The larger operand's tiles are the slower dimension of the order.
+    const bool mFast = static_cast<uint64_t>(rows) * 4 <= static_cast<uint64_t>(virtualRows) * 2;
+    const GemmOrder order{CeilDiv(rows, kGemmTiles[best].bm), CeilDiv(virtualRows, kGemmTiles[best].bn), mFast};
+    const uint64_t blocks = static_cast<uint64_t>(order.mTiles) * order.nTiles * splits;
+    if (blocks > std::numeric_limits<int32_t>::max())
+    {
+        return hipErrorInvalidValue;
+    }
+    const uint32_t kPerSplit = ColumnsPerSplit(k, splits);
+    switch (best)
+    {
+#define MUYO_GEMM_LAUNCH(I, WM, WN, WK, MB, NB, ST, BK, PER)                                                           \
+    case I:                                                                                                            \
+    {                                                                                                                  \
+        using T = GemmTile<WM, WN, WK, MB, NB, ST, BK, PER>;                                                           \
+        static_assert(T::kBm == kGemmTiles[I].bm && T::kBn == kGemmTiles[I].bn && BK == kGemmTiles[I].bk &&            \
+                          ST == kGemmTiles[I].stages && PER == kGemmTiles[I].perCu,                                    \
+                      "kGemmTiles");                                                                                   \
+        hipLaunchKernelGGL((GemmSplitKernel<T, WM, WN, WK, MB, NB, ST, BK, Epi>), dim3(static_cast<uint32_t>(blocks)), \
+                           dim3(T::kThreads), 0, s, ahi, alo, epi, rows, k, kPerSplit, order);                         \
+        break;                                                                                                         \
+    }
+        MUYO_GEMM_TILES(MUYO_GEMM_LAUNCH)
+#undef MUYO_GEMM_LAUNCH
+        default:
+            return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+}  // namespace
+
+uint32_t GemmSplits(uint32_t rows, uint32_t n, uint32_t k)
+{
+    uint32_t best = 1;
+    double bestCost = std::numeric_limits<double>::infinity();
+    for (uint32_t splits = 1; splits <= MaxGemmSplits(rows) && rows > 0 && n > 0 && k > 0; ++splits)
+    {
+        // Splits of whole kGemmSplitUnits, none of them empty.
+        if (CeilDiv(k, ColumnsPerSplit(k, splits)) != splits)
+        {
+            continue;
+        }
+        for (const GemmTileCost& tile : kGemmTiles)
+        {
+            const double cost = GemmCost(tile, rows, n, k, splits);
+            if (cost < bestCost)
+            {
+                bestCost = cost;
+                best = splits;
+            }
+        }
+    }
+    return best;
+}
+
+hipError_t LaunchGemmSplit(hipStream_t s, const uint16_t* ahi, const uint16_t* alo, const uint16_t* w,
+                           const float* bias, const float* residual, float* out, uint32_t rows, uint32_t n,
+                           uint32_t k, float* partial, uint32_t splits)
+{
+    if (n % 4 != 0 || k % 8 != 0 || splits == 0 || splits > kMaxGemmSplits || (splits > 1 && partial == nullptr))
+    {
+        return hipErrorInvalidValue;
+    }
+    PlainEpi epi{w, bias, residual, out, n, k};
+    epi.partial = splits > 1 ? partial : nullptr;
+    return LaunchGemm(s, ahi, alo, epi, rows, n, k, splits);
+}
+
+hipError_t LaunchGemmSwiGlu(hipStream_t s, const uint16_t* ahi, const uint16_t* alo, const uint16_t* wgate,
+                            const uint16_t* wup, uint16_t* hhi, uint16_t* hlo, uint32_t rows, uint32_t ffn,
+                            uint32_t k)
+{
+    if (ffn % 4 != 0 || k % 8 != 0)
+    {
+        return hipErrorInvalidValue;
+    }
+    // Two virtual rows (gate, up) per output, in whole 32-row blocks.
+    const uint32_t virtualRows = 2 * CeilDiv(ffn, 16) * 16;
+    return LaunchGemm(s, ahi, alo, SwiGluEpi{wgate, wup, hhi, hlo, ffn, k}, rows, virtualRows, k);
+}
+}  // namespace muyo

@@ -221,6 +221,50 @@ def test_gemm_swiglu_matches_per_token_path(mh, gpu, orc, rows, ffn, k):
     assert worst(got, want) < 2e-5
 
 
+# Each tile shape of the GEMM at a size that selects it, one past a whole tile in rows or weight
+# rows, with a K that ends inside a slab and inside a 16-column step.
+TILE_SHAPES = [
+    (980, 13420, 264),   # 256 x 256
+    (208, 21076, 264),   # 128 x 192
+    (1541, 1364, 264),   # 64 x 256
+    (1, 33592, 536),     # 64 x 192
+    (65, 9732, 280),     # 32 x 128, two workgroups per CU
+    (33, 9092, 904),     # 32 x 128, 128-column slabs
+    (33, 132, 584),      # 32 x 64
+    (1, 4, 8),
+]
+
+
+@pytest.mark.parametrize("rows,n,k", TILE_SHAPES)
+def test_gemm_tile_shapes_exact_with_both_planes(mh, gpu, rows, n, k):
+    """Values whose products and sums are exact in f32 (hi and weights integers up to 2, lo a
+    multiple of 2^-10: at most 11 + 1 + 10 bits), so the plain GEMM must match to the bit and the
+    swiglu GEMM to the planes' precision."""
+    torch = gpu
+    g = torch.Generator(device="cuda").manual_seed(rows * 31 + n + k)
+
+    def ints(shape, scale=1.0):
+        return (torch.randint(-2, 3, shape, device="cuda", generator=g) * scale).to(torch.float16)
+
+    hi, lo, w = ints((rows, k)), ints((rows, k), 2.0 ** -11), ints((n, k))
+    lib = mh.load()
+    out = torch.full((rows, n), float("nan"), dtype=torch.float32, device="cuda")
+    run(mh, torch, lib.muyo_gemm_split_f16(hi.data_ptr(), lo.data_ptr(), w.data_ptr(), None, None, out.data_ptr(),
+                                           rows, n, k, stream(torch)))
+    a = hi.double() + lo.double()
+    assert torch.equal(out.double(), a @ w.double().t().contiguous())
+    ffn = n // 8 * 4 or 4
+    gate, up = ints((ffn, k)), ints((ffn, k))
+    hhi, hlo = planes(torch, (rows, ffn))
+    run(mh, torch, lib.muyo_gemm_swiglu_split_f16(hi.data_ptr(), lo.data_ptr(), gate.data_ptr(), up.data_ptr(),
+                                                  hhi.data_ptr(), hlo.data_ptr(), rows, ffn, k, stream(torch)))
+    gv, uv = a @ gate.double().t().contiguous(), a @ up.double().t().contiguous()
+    want = gv * torch.sigmoid(gv) * uv
+    got = hhi.view(torch.float16).double() + hlo.view(torch.float16).double()
+    # The planes hold 21 bits of each value, and expf and the division are within a few ulp.
+    assert float((got - want).abs().max()) <= 2e-6 * float(1 + want.abs().max())
+
+
 def test_gemm_refusals(mh, gpu):
     lib = mh.load()
     fake = ctypes.c_void_p(256)
