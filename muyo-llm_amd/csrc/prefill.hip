@@ -464,351 +464,6 @@ __global__ __launch_bounds__(256) void RopeSplitAppendQuadKernel(const float* __
     }
 }
 
-// ------------------------------------------------------------------------------------------------
-// Causal flash attention. A workgroup owns one kv head, 32 consecutive queries and up to
-// kHeadsPerBlock of the group's query heads, one per wave (a group of 7 takes two workgroups when
-// one per tile would leave CUs idle); the waves share each 32-key tile of K and V through LDS (V
-// stored transposed, channel-major). The next tile's rows are loaded into registers while the
-// current one is multiplied, so a workgroup waits on memory once, not once per tile. Per wave
-// and tile:
-//   S^T (keys x queries) = K . Q^T on the matrix cores (K the A operand from LDS, Q the B operand
-//   held in registers as split planes), so a lane holds 16 keys of one query and the online
-//   softmax needs only one exchange with the lane 32 away;
-//   O^T (channels x queries) += V^T . P^T with P^T split into planes straight from the S^T
-//   accumulators: the B operand's k slot (h, v) of lane j + 32h is key 16 s + 8 (v / 4) + 4 h +
-//   v % 4 of the tile, and the V^T fragment reads the same keys (two 8-byte LDS reads).
-
-constexpr int kAttnKeys = 32;
-constexpr uint32_t kAttnChunkTiles = 16;  // key tiles per chunk of a split query tile, at least
-
-/// Key tiles (of kAttnKeys) a query tile attends to: cache rows 0 .. its last query's position.
-__host__ __device__ inline uint32_t AttnKeyTiles(uint32_t qtile, uint32_t rows, int32_t pos0)
-{
-    const uint32_t last = qtile * 32 + 31 < rows ? qtile * 32 + 31 : rows - 1;
-    return (static_cast<uint32_t>(pos0) + last) / kAttnKeys + 1;
-}
-
-/// Work items of the split prefill attention, passed by value in the kernel arguments.
-struct AttnWork
-{
-    uint32_t count;       // items; 0: one item per query tile over all of its keys
-    uint32_t chunkTiles;  // key tiles per chunk
-    uint16_t tile[kAttnMaxItems];
-    uint8_t chunk[kAttnMaxItems];
-};
-
-/// Softmax partials of the chunks of split tiles: [kAttnMaxChunks][rows][heads] (running max in
-/// log2 units, sum) and [kAttnMaxChunks][rows][heads][headDim] (unnormalised P.V).
-struct AttnPartials
-{
-    float* max;
-    float* sum;
-    float* acc;
-};
-
-/// Combines the chunk partials of the split tiles' queries into their output planes: out = sum_c
-/// 2^(m_c - M) acc_c / sum_c 2^(m_c - M) l_c, M the largest m_c (a chunk with no key of the query
-/// weighs 0). A thread per (query, head, 4 channels); queries of unsplit tiles are left alone.
-__global__ __launch_bounds__(256) void PrefillAttnMergeKernel(AttnPartials part, uint16_t* __restrict__ ohi,
-                                                              uint16_t* __restrict__ olo, uint32_t rows, int32_t pos0,
-                                                              uint32_t heads, uint32_t headDim, uint32_t chunkTiles)
-{
-    const uint32_t quads = headDim / 4;
-    const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= static_cast<uint64_t>(rows) * heads * quads)
-    {
-        return;
-    }
-    const uint32_t channel = static_cast<uint32_t>(i % quads) * 4;
-    const uint32_t head = static_cast<uint32_t>(i / quads % heads);
-    const uint32_t m = static_cast<uint32_t>(i / quads / heads);
-    const uint32_t keyTiles = AttnKeyTiles(m / 32, rows, pos0);
-    if (keyTiles <= chunkTiles)
-    {
-        return;
-    }
-    const uint32_t chunks = (keyTiles + chunkTiles - 1) / chunkTiles;
-    // Every slot's operands requested at once (slots past `chunks` reread slot 0 and weigh 0).
-    float mc[kAttnMaxChunks];
-    float lc[kAttnMaxChunks];
-    float4 ac[kAttnMaxChunks];
-#pragma unroll
-    for (uint32_t c = 0; c < kAttnMaxChunks; ++c)
-    {
-        const uint64_t at = (static_cast<uint64_t>(c < chunks ? c : 0) * rows + m) * heads + head;
-        mc[c] = part.max[at];
-        lc[c] = part.sum[at];
-        ac[c] = *reinterpret_cast<const float4*>(part.acc + at * headDim + channel);
-    }
-    float top = -INFINITY;
-#pragma unroll
-    for (uint32_t c = 0; c < kAttnMaxChunks; ++c)
-    {
-        top = c < chunks ? fmaxf(top, mc[c]) : top;
-    }
-    float den = 0.0f;
-    float4 num = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-#pragma unroll
-    for (uint32_t c = 0; c < kAttnMaxChunks; ++c)
-    {
-        if (c < chunks)
-        {
-            const float w = mc[c] == -INFINITY ? 0.0f : exp2f(mc[c] - top);
-            den = fmaf(w, lc[c], den);
-            num.x = fmaf(w, ac[c].x, num.x);
-            num.y = fmaf(w, ac[c].y, num.y);
-            num.z = fmaf(w, ac[c].z, num.z);
-            num.w = fmaf(w, ac[c].w, num.w);
-        }
-    }
-    const float inv = 1.0f / den;
-    StoreSplit4(ohi, olo, static_cast<uint64_t>(m) * heads * headDim + head * headDim + channel, num.x * inv,
-                num.y * inv, num.z * inv, num.w * inv);
-}
-// Halves per transposed V row. The even lane of each key pair stores both keys of a channel as one
-// 4-byte word, so the 16 storing lanes of a channel chunk write 64 contiguous bytes; 36 halves
-// (18 words) put the two chunks a wave stores at once 16 banks apart, and the MFMA fragment reads
-// of 32 consecutive rows (8 bytes each, 18 words apart) cover every bank once.
-constexpr int kVStride = kAttnKeys + 4;
-
-/// Grid (head splits, work items, kv heads): the splits of one item are dispatched together.
-/// Without work items (work.count 0) item y is query tile tiles - 1 - y over all of its keys (the
-/// longest tiles first) and writes the output planes. With them, item y is query tile
-/// work.tile[y] over key tiles [c * C, (c + 1) * C) of its range (c = work.chunk[y],
-/// C = work.chunkTiles); a tile split over several chunks leaves each chunk's unnormalised
-/// softmax partial (running max, sum, P.V) in slot c of `part` for PrefillAttnMergeKernel, a tile
-/// of one chunk writes its planes directly. A causal tile's key range grows with its position, so
-/// the split evens the workgroups' work: a 2048-token prompt is 64 tiles of 1..64 key tiles.
-template <int kHd, int kHeadsPerBlock>
-__global__ __launch_bounds__(kWave * kHeadsPerBlock) void PrefillAttentionKernel(
-    const uint16_t* __restrict__ qhi, const uint16_t* __restrict__ qlo, const uint16_t* __restrict__ kcache,
-    const uint16_t* __restrict__ vcache, uint16_t* __restrict__ ohi, uint16_t* __restrict__ olo, uint32_t rows,
-    int32_t pos0, uint32_t heads, uint32_t kvHeads, uint32_t maxSeq, float scale, AttnWork work, AttnPartials part)
-{
-    constexpr int kKStride = kHd + 8;
-    constexpr int kChunks = kHd / 8;
-    constexpr int kThreads = kWave * kHeadsPerBlock;
-    constexpr int kLoads = (kAttnKeys * kChunks + kThreads - 1) / kThreads;  // K (and V) chunks per thread per tile
-    __shared__ __attribute__((aligned(16))) uint16_t kTile[kAttnKeys * kKStride];
-    __shared__ __attribute__((aligned(16))) uint16_t vTile[kHd * kVStride];
-
-    const uint32_t group = heads / kvHeads;
-    const bool itemized = work.count > 0;
-    const uint32_t qtile = itemized ? work.tile[blockIdx.y] : gridDim.y - 1 - blockIdx.y;  // longest first
-    const uint32_t g = blockIdx.z;
-    const uint32_t wave = threadIdx.x / kWave;
-    const uint32_t lane = threadIdx.x % kWave;
-    const uint32_t h = lane / 32;
-    const uint32_t inGroup = blockIdx.x * kHeadsPerBlock + wave;
-    const bool active = inGroup < group;  // a wave past the group only loads tiles
-    const uint32_t head = g * group + (active ? inGroup : group - 1);
-    const uint32_t qdim = heads * kHd;
-    const uint32_t m0 = qtile * 32;
-    const uint32_t mq = m0 + lane % 32 < rows ? m0 + lane % 32 : rows - 1;
-    const int32_t qpos = pos0 + static_cast<int32_t>(mq);
-    const int32_t lastPos = pos0 + static_cast<int32_t>(m0 + 31 < rows ? m0 + 31 : rows - 1);
-    const uint32_t keyTiles = AttnKeyTiles(qtile, rows, pos0);
-    const uint32_t chunk = itemized ? work.chunk[blockIdx.y] : 0;
-    const uint32_t ktBegin = itemized ? chunk * work.chunkTiles : 0;
-    const uint32_t ktEnd = itemized ? min(keyTiles, ktBegin + work.chunkTiles) : keyTiles;
-    const bool partial = itemized && keyTiles > work.chunkTiles;  // the tile spans several chunks
-
-    half8 qh[kHd / 16], ql[kHd / 16];
-    {
-        const uint64_t at = static_cast<uint64_t>(mq) * qdim + head * kHd + 8 * h;
-#pragma unroll
-        for (int s = 0; s < kHd / 16; ++s)
-        {
-            qh[s] = *reinterpret_cast<const half8*>(qhi + at + 16 * s);
-            ql[s] = *reinterpret_cast<const half8*>(qlo + at + 16 * s);
-        }
-    }
-    floatx16 o[kHd / 32];
-#pragma unroll
-    for (int c = 0; c < kHd / 32; ++c)
-    {
-        o[c] = floatx16{};
-    }
-    float runMax = -INFINITY;  // log2 units: scores scaled by log2(e), weights 2^(s - max)
-    float runSum = 0.0f;
-    const float scaleLog2 = scale * 1.44269504088896340736f;
-    const uint16_t* kBase = kcache + static_cast<uint64_t>(g) * maxSeq * kHd;
-    const uint16_t* vBase = vcache + static_cast<uint64_t>(g) * maxSeq * kHd;
-
-    half8 kReg[kLoads], vReg[kLoads];
-    auto loadTile = [&](uint32_t kt) {
-#pragma unroll
-        for (int i = 0; i < kLoads; ++i)
-        {
-            const uint32_t c = threadIdx.x + i * kThreads;
-            const uint32_t r = c % kAttnKeys;               // key within the tile
-            const uint32_t cc = (c / kAttnKeys) % kChunks;  // 8-channel chunk
-            const uint32_t key = kt * kAttnKeys + r < maxSeq ? kt * kAttnKeys + r : maxSeq - 1;
-            kReg[i] = *reinterpret_cast<const half8*>(kBase + static_cast<uint64_t>(key) * kHd + cc * 8);
-            vReg[i] = *reinterpret_cast<const half8*>(vBase + static_cast<uint64_t>(key) * kHd + cc * 8);
-        }
-    };
-    loadTile(ktBegin);
-    for (uint32_t kt = ktBegin; kt < ktEnd; ++kt)
-    {
-        __syncthreads();  // every wave is done with the previous tile
-#pragma unroll
-        for (int i = 0; i < kLoads; ++i)
-        {
-            const uint32_t c = threadIdx.x + i * kThreads;
-            if (c < kAttnKeys * kChunks)
-            {
-                const uint32_t r = c % kAttnKeys;
-                const uint32_t cc = c / kAttnKeys;
-                *reinterpret_cast<half8*>(kTile + r * kKStride + cc * 8) = kReg[i];
-            }
-            // Rows past the tile's last query position may hold anything (NaN, inf): their weight
-            // is 0, and 0 * NaN would poison every query of the tile, so they enter the V tile as
-            // zeros. Their scores are masked to -inf by position. Lanes hold consecutive keys of a
-            // chunk (c % 32), so the odd lane's row reaches its even partner by a quad permute
-            // (lanes swapped in pairs) and the even lane stores both keys of each channel.
-            const uint32_t r = c % kAttnKeys;
-            const uint32_t cc = (c / kAttnKeys) % kChunks;
-            const bool live = static_cast<int32_t>(kt * kAttnKeys + r) <= lastPos;
-            const half8 v = live ? vReg[i] : half8{};
-            uint32_t mine[4];
-            __builtin_memcpy(mine, &v, sizeof(mine));
-            uint32_t other[4];
-#pragma unroll
-            for (int d = 0; d < 4; ++d)
-            {
-                other[d] = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
-                    static_cast<int>(mine[d]), static_cast<int>(mine[d]), 0xB1, 0xF, 0xF, false));
-            }
-            if (c < kAttnKeys * kChunks && (r & 1u) == 0)
-            {
-                uint32_t* row = reinterpret_cast<uint32_t*>(vTile) + ((cc * 8) * kVStride + r) / 2;
-#pragma unroll
-                for (int d = 0; d < 4; ++d)
-                {
-                    // Channel 2d: the low halves of this key and the next; channel 2d + 1: the high.
-                    row[(2 * d) * (kVStride / 2)] = (mine[d] & 0xFFFFu) | (other[d] << 16);
-                    row[(2 * d + 1) * (kVStride / 2)] = (mine[d] >> 16) | (other[d] & 0xFFFF0000u);
-                }
-            }
-        }
-        __syncthreads();
-        if (kt + 1 < ktEnd)
-        {
-            loadTile(kt + 1);  // in flight while this tile is multiplied
-        }
-        if (!active)
-        {
-            continue;
-        }
-
-        floatx16 st = floatx16{};
-        const uint16_t* kFrag = kTile + (lane % 32) * kKStride + 8 * h;
-#pragma unroll
-        for (int s = 0; s < kHd / 16; ++s)
-        {
-            const half8 kf = *reinterpret_cast<const half8*>(kFrag + 16 * s);
-            st = Mfma(kf, qh[s], st);
-            st = Mfma(kf, ql[s], st);
-        }
-        float p[16];
-        float tileMax = -INFINITY;
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-        {
-            const int32_t key = static_cast<int32_t>(kt * kAttnKeys + 8 * (r / 4) + 4 * h + r % 4);
-            p[r] = key <= qpos ? st[r] * scaleLog2 : -INFINITY;
-            tileMax = fmaxf(tileMax, p[r]);
-        }
-        tileMax = fmaxf(tileMax, __shfl_xor(tileMax, 32));
-        // Finite over a query's whole range (key 0 is in it), but a chunk of a split tile may hold
-        // no key of a query yet: then nothing accumulates (factor 1, weights 0).
-        const float newMax = fmaxf(runMax, tileMax);
-        const bool none = newMax == -INFINITY;
-        const float factor = none ? 1.0f : exp2f(runMax - newMax);
-        float sum = 0.0f;
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-        {
-            p[r] = none ? 0.0f : exp2f(p[r] - newMax);
-            sum += p[r];
-        }
-        runSum = runSum * factor + sum;
-        runMax = newMax;
-#pragma unroll
-        for (int c = 0; c < kHd / 32; ++c)
-        {
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-            {
-                o[c][r] *= factor;
-            }
-        }
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-        {
-            half8 ph, pl;
-#pragma unroll
-            for (int v = 0; v < 8; ++v)
-            {
-                ph[v] = HiHalf(p[8 * s + v]);
-                pl[v] = LoHalf(p[8 * s + v]);
-            }
-#pragma unroll
-            for (int c = 0; c < kHd / 32; ++c)
-            {
-                const _Float16* row =
-                    reinterpret_cast<const _Float16*>(vTile) + (c * 32 + lane % 32) * kVStride + 16 * s + 4 * h;
-                const half4 v0 = *reinterpret_cast<const half4*>(row);
-                const half4 v1 = *reinterpret_cast<const half4*>(row + 8);
-                const half8 vf = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
-                o[c] = Mfma(vf, ph, o[c]);
-                o[c] = Mfma(vf, pl, o[c]);
-            }
-        }
-    }
-
-    const float total = runSum + __shfl_xor(runSum, 32);
-    const uint32_t m = m0 + lane % 32;
-    if (active && m < rows && partial)
-    {
-        // Slot `chunk`: the running max and sum of the query (both halves of the wave agree on
-        // the max; their sums are added), and its unnormalised P.V.
-        const uint64_t at = (static_cast<uint64_t>(chunk) * rows + m) * heads + head;
-        if (h == 0)
-        {
-            part.max[at] = runMax;
-            part.sum[at] = total;
-        }
-#pragma unroll
-        for (int c = 0; c < kHd / 32; ++c)
-        {
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-            {
-                const uint32_t channel = c * 32 + 8 * q + 4 * h;
-                *reinterpret_cast<float4*>(part.acc + at * kHd + channel) =
-                    make_float4(o[c][4 * q], o[c][4 * q + 1], o[c][4 * q + 2], o[c][4 * q + 3]);
-            }
-        }
-    }
-    else if (active && m < rows)
-    {
-        const float inv = 1.0f / total;
-        const uint64_t base = static_cast<uint64_t>(m) * qdim + head * kHd;
-#pragma unroll
-        for (int c = 0; c < kHd / 32; ++c)
-        {
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-            {
-                const uint32_t channel = c * 32 + 8 * q + 4 * h;
-                StoreSplit4(ohi, olo, base + channel, o[c][4 * q] * inv, o[c][4 * q + 1] * inv,
-                            o[c][4 * q + 2] * inv, o[c][4 * q + 3] * inv);
-            }
-        }
-    }
-}
 }  // namespace
 
 hipError_t LaunchEmbedRows(hipStream_t s, const uint16_t* table, const int32_t* tokens, uint32_t rows,
@@ -877,93 +532,6 @@ hipError_t LaunchRopeSplitAppend(hipStream_t s, const float* qkv, uint32_t rows,
     hipLaunchKernelGGL(RopeSplitAppendKernel, dim3(CeilDiv(total, 256)), dim3(256), 0, s, qkv, rows, pos0, heads,
                        kvHeads, headDim, maxSeq, ropePow, qhi, qlo, kcache, vcache, splits, bias);
     return hipGetLastError();
-}
-
-hipError_t LaunchPrefillAttention(hipStream_t s, const uint16_t* qhi, const uint16_t* qlo, const uint16_t* kcache,
-                                  const uint16_t* vcache, uint16_t* ohi, uint16_t* olo, uint32_t rows, int32_t pos0,
-                                  uint32_t heads, uint32_t kvHeads, uint32_t headDim, uint32_t maxSeq, float scale,
-                                  float* workspace, size_t workspaceFloats)
-{
-    if (rows == 0 || kvHeads == 0 || heads % kvHeads != 0 || heads / kvHeads > 8 || pos0 < 0 ||
-        static_cast<uint64_t>(pos0) + rows > maxSeq)
-    {
-        return hipErrorInvalidValue;
-    }
-    // A workgroup per (kv head, query tile) holding the whole group when that alone fills the chip
-    // (7B shape: 256 workgroups, one K/V staging per tile for all 7 heads); otherwise groups past
-    // four heads take two workgroups (0.5B shape: 128 -> 256).
-    const uint32_t group = heads / kvHeads;
-    int device = 0;
-    int cus = 256;
-    if (hipGetDevice(&device) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
-    {
-        cus = 256;
-    }
-    const uint32_t tiles = CeilDiv(rows, 32);
-    const bool fills = static_cast<uint64_t>(tiles) * kvHeads >= static_cast<uint64_t>(cus);
-    const uint32_t perBlock = group <= 1 ? 1 : group <= 2 ? 2 : group <= 4 || !fills ? 4 : 8;
-    // Split the long tiles' key ranges into chunks of at least kAttnChunkTiles key tiles (and at
-    // most kAttnMaxChunks per tile), items ordered longest first. Prompts whose chunks would not
-    // fit kAttnMaxItems (past 2048 queries) run unsplit.
-    AttnWork work{};
-    AttnPartials part{};
-    const uint32_t longest = AttnKeyTiles(tiles - 1, rows, pos0);
-    const uint32_t chunkTiles = std::max(kAttnChunkTiles, CeilDiv(longest, kAttnMaxChunks));
-    uint64_t items = 0;
-    for (uint32_t t = 0; t < tiles; ++t)
-    {
-        items += CeilDiv(AttnKeyTiles(t, rows, pos0), chunkTiles);
-    }
-    if (workspace != nullptr && workspaceFloats >= PrefillAttentionWorkspaceFloats(rows, heads, headDim) &&
-        longest > chunkTiles && items <= kAttnMaxItems)
-    {
-        work.chunkTiles = chunkTiles;
-        for (uint32_t len = chunkTiles; len > 0 && work.count < kAttnMaxItems; --len)
-        {
-            for (uint32_t t = tiles; t-- > 0;)
-            {
-                const uint32_t keyTiles = AttnKeyTiles(t, rows, pos0);
-                for (uint32_t c = 0; c * chunkTiles < keyTiles; ++c)
-                {
-                    if (std::min(chunkTiles, keyTiles - c * chunkTiles) == len && work.count < kAttnMaxItems)
-                    {
-                        work.tile[work.count] = static_cast<uint16_t>(t);
-                        work.chunk[work.count] = static_cast<uint8_t>(c);
-                        ++work.count;
-                    }
-                }
-            }
-        }
-        const size_t stats = static_cast<size_t>(kAttnMaxChunks) * rows * heads;
-        part = AttnPartials{workspace, workspace + stats, workspace + 2 * stats};
-    }
-    const dim3 grid(CeilDiv(group, perBlock), work.count > 0 ? work.count : tiles, kvHeads);
-    const dim3 block(kWave * perBlock);
-#define MUYO_PREFILL_ATTENTION(HD, P)                                                                         \
-    if (headDim == HD && perBlock == P)                                                                       \
-    {                                                                                                         \
-        hipLaunchKernelGGL((PrefillAttentionKernel<HD, P>), grid, block, 0, s, qhi, qlo, kcache, vcache, ohi,  \
-                           olo, rows, pos0, heads, kvHeads, maxSeq, scale, work, part);                       \
-        if (work.count == 0)                                                                                  \
-        {                                                                                                     \
-            return hipGetLastError();                                                                         \
-        }                                                                                                     \
-        const uint64_t threads = static_cast<uint64_t>(rows) * heads * (headDim / 4);                         \
-        hipLaunchKernelGGL(PrefillAttnMergeKernel, dim3(static_cast<uint32_t>(CeilDiv(threads, 256))),        \
-                           dim3(256), 0, s, part, ohi, olo, rows, pos0, heads, headDim, work.chunkTiles);      \
-        return hipGetLastError();                                                                             \
-    }
-    MUYO_PREFILL_ATTENTION(64, 1)
-    MUYO_PREFILL_ATTENTION(64, 2)
-    MUYO_PREFILL_ATTENTION(64, 4)
-    MUYO_PREFILL_ATTENTION(64, 8)
-    MUYO_PREFILL_ATTENTION(128, 1)
-    MUYO_PREFILL_ATTENTION(128, 2)
-    MUYO_PREFILL_ATTENTION(128, 4)
-    MUYO_PREFILL_ATTENTION(128, 8)
-#undef MUYO_PREFILL_ATTENTION
-    return hipErrorInvalidValue;
 }
 }  // namespace muyo
 

@@ -39,8 +39,7 @@ inline size_t GemmPartialFloats(uint32_t rows, uint32_t n)
     const size_t many = static_cast<size_t>(kMaxGemmSplits / 2) * rows;
     return (few > many ? few : many) * n;
 }
-constexpr uint32_t kAttnMaxChunks = 8;    // key chunks a split prefill-attention query tile takes at most
-constexpr uint32_t kAttnMaxItems = 512;   // work items of one split attention launch (64 tiles x 8)
+constexpr uint32_t kAttnMaxChunks = 8;  // key chunks a split prefill-attention query tile takes at most
 
 /// Floats of the workspace the split prefill attention needs for `rows` queries.
 inline size_t PrefillAttentionWorkspaceFloats(uint32_t rows, uint32_t heads, uint32_t headDim)

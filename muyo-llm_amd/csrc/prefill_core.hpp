@@ -39,4 +39,11 @@ __device__ __forceinline__ void StoreSplit4(uint16_t* hi, uint16_t* lo, uint64_t
     *reinterpret_cast<half4*>(hi + at) = h;
     *reinterpret_cast<half4*>(lo + at) = l;
 }
+/// Waits until at most kLeft of this wave's loads are in flight and its LDS reads are done, then
+/// meets the other waves.
+template <int kLeft>
+__device__ __forceinline__ void WaitAndMeet()
+{
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kLeft) : "memory");
+}
 }  // namespace muyo

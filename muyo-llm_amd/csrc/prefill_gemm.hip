@@ -150,14 +150,6 @@ struct SwiGluEpi
     }
 };
 
-/// Waits until at most kLeft of this wave's loads are in flight and its LDS reads are done, then
-/// meets the other waves.
-template <int kLeft>
-__device__ __forceinline__ void WaitAndMeet()
-{
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kLeft) : "memory");
-}
-
 /// A tile of kBm tokens x kBn weight rows by kWm x kWn x kWk waves: a wave owns kMb x kNb blocks
 /// of 32 x 32 outputs, and with kWk > 1 that many waves own the same blocks and every kWk-th step
 /// of 16 columns, their sums meeting in LDS at the end.

@@ -415,6 +415,53 @@ def test_prefill_attention_key_chunks_ignore_rows_past_the_prompt(mh, gpu, orc, 
                            split=True)
 
 
+@pytest.mark.parametrize("heads,kv_heads,head_dim,rows,pos0,max_seq,scale,spread", [
+    (14, 2, 64, 37, 91, 129, 0.125, 1.0),     # group of 7 over two query tiles, an odd cache end
+    (4, 4, 64, 130, 0, 130, 0.125, 30.0),     # no grouping; maxima that rise past the 2^8 slack
+    (28, 4, 128, 65, 63, 133, 0.088, 1.0),    # a step's edge inside the prompt
+    (6, 2, 128, 33, 2000, 2047, 0.3, 30.0),   # chunks, peaked
+    (16, 2, 128, 1, 0, 1, 0.088, 1.0),        # one key
+    (8, 1, 64, 40, 700, 741, -0.2, 2.0),      # a negative scale
+    (3, 1, 128, 70, 10, 100, 0.0, 1.0),       # every key the same weight
+])
+@pytest.mark.parametrize("workspace", [False, True])
+def test_prefill_attention_edges_against_float64(mh, gpu, heads, kv_heads, head_dim, rows, pos0, max_seq, scale,
+                                                 spread, workspace):
+    """Query tiles, key steps, chunks, cache ends and scales at their edges against float64. The rows
+    of the cache past the prompt hold NaN. Tolerance: weights and queries carry 21 bits, sums are
+    f32 over at most 1024 keys a chunk (measured below 1e-6 of the result's norm)."""
+    torch = gpu
+    g = torch.Generator(device="cuda").manual_seed(heads * 1000 + rows)
+    q = torch.randn((rows, heads, head_dim), device="cuda", generator=g) * spread
+    cache = [torch.randn((kv_heads, max_seq, head_dim), device="cuda", generator=g).half() for _ in range(2)]
+    for c in cache:
+        c[:, pos0 + rows:] = float("nan")
+    qhi = q.half()
+    qlo = (q - qhi.float()).half()
+    ohi, olo = planes(torch, (rows, heads * head_dim))
+    lib = mh.load()
+    args = (qhi.data_ptr(), qlo.data_ptr(), cache[0].data_ptr(), cache[1].data_ptr(), ohi.data_ptr(), olo.data_ptr(),
+            rows, pos0, heads, kv_heads, head_dim, max_seq, scale)
+    if workspace:
+        size = lib.muyo_prefill_attention_workspace_bytes(rows, heads, head_dim)
+        space = torch.full((size // 4,), float("nan"), device="cuda")
+        run(mh, torch, lib.muyo_prefill_attention_f16kv_ws(*args, space.data_ptr(), size, stream(torch)))
+    else:
+        run(mh, torch, lib.muyo_prefill_attention_f16kv(*args, stream(torch)))
+    qq = qhi.double() + qlo.double()
+    keys = pos0 + rows
+    late = torch.arange(keys, device="cuda")[None] > torch.arange(pos0, keys, device="cuda")[:, None]
+    want = torch.empty_like(qq)
+    for h in range(heads):
+        k, v = (c[h // (heads // kv_heads), :keys].double() for c in cache)
+        score = (qq[:, h] @ k.t().contiguous()) * float(np.float32(scale))
+        want[:, h] = torch.softmax(score.masked_fill_(late, -math.inf), -1) @ v
+    got = (ohi.view(torch.float16).double() + olo.view(torch.float16).double()).view(rows, heads, head_dim)
+    # Scores of magnitude s carry s * 2^-22 from q's planes and the f32 sums into the exponent.
+    top = float((qq.norm(dim=-1).max() * cache[0][:, :keys].double().norm(dim=-1).max()) * abs(scale))
+    assert float((got - want).norm() / want.norm()) <= 2e-6 + top * 2.0 ** -22
+
+
 def test_prefill_attention_refusals(mh, gpu):
     lib = mh.load()
     fake = ctypes.c_void_p(256)
