@@ -521,11 +521,18 @@ struct ArgMaxArgs
     uint32_t gx, gy, gz;
 };
 
-__global__ __launch_bounds__(kBlock) void ArgMaxRows(const float* __restrict__ a, int32_t* __restrict__ d,
-                                                     ArgMaxArgs p)
+/// One row by a workgroup of kThreads, each with kDepth 16-byte loads in flight. With a workgroup per
+/// CU or fewer, nothing else hides a row's latency: 256 threads of four loads (16 KB in flight) take
+/// 38 round trips over a row of 151936, 20.1 us where the LM head has just written it; 1024 threads
+/// of eight take five, about 10 us. Batches of many rows keep the small workgroups, whose number
+/// hides it. (Splitting a row over workgroups without a workspace, each exchanging its index into d
+/// atomically, took 7.1 us for one row but 45 against 20 for 64: the exchanges queue.)
+template <int kThreads, int kDepth>
+__global__ __launch_bounds__(kThreads) void ArgMaxRows(const float* __restrict__ a, int32_t* __restrict__ d,
+                                                       ArgMaxArgs p)
 {
-    __shared__ float bestValue[kWaves];
-    __shared__ int32_t bestIndex[kWaves];
+    __shared__ float bestValue[kThreads / kWave];
+    __shared__ int32_t bestIndex[kThreads / kWave];
     uint32_t row;
     SlotRow(blockIdx.x, p.gx, p.gy, row);
     if (row >= p.ky)
@@ -542,28 +549,28 @@ __global__ __launch_bounds__(kBlock) void ArgMaxRows(const float* __restrict__ a
         const uint32_t n4 = p.kx / 4;
         const float4v* x4 = reinterpret_cast<const float4v*>(x);
         uint32_t i = threadIdx.x;
-        // Four non-temporal loads in flight per thread, taken in index order (4096 x 151936:
-        // 6.1 -> 6.9 TB/s against one load at a time).
-        for (; i + 3 * kBlock < n4; i += 4 * kBlock)
+        // kDepth non-temporal loads in flight per thread, taken in index order (4096 x 151936:
+        // 6.1 -> 6.9 TB/s with four against one load at a time).
+        for (; i + (kDepth - 1) * kThreads < n4; i += kDepth * kThreads)
         {
-            float4v v[4];
+            float4v v[kDepth];
 #pragma unroll
-            for (int k = 0; k < 4; ++k)
+            for (int k = 0; k < kDepth; ++k)
             {
-                v[k] = __builtin_nontemporal_load(x4 + i + k * kBlock);
+                v[k] = __builtin_nontemporal_load(x4 + i + k * kThreads);
             }
 #pragma unroll
-            for (int k = 0; k < 4; ++k)
+            for (int k = 0; k < kDepth; ++k)
             {
                 // Within one thread indices only grow, so strict '>' keeps the lowest on ties.
-                const int32_t base = static_cast<int32_t>((i + k * kBlock) * 4);
+                const int32_t base = static_cast<int32_t>((i + k * kThreads) * 4);
                 if (v[k].x > value) { value = v[k].x; index = base; }
                 if (v[k].y > value) { value = v[k].y; index = base + 1; }
                 if (v[k].z > value) { value = v[k].z; index = base + 2; }
                 if (v[k].w > value) { value = v[k].w; index = base + 3; }
             }
         }
-        for (; i < n4; i += kBlock)
+        for (; i < n4; i += kThreads)
         {
             const float4v v = __builtin_nontemporal_load(x4 + i);
             const int32_t base = static_cast<int32_t>(i * 4);
@@ -574,7 +581,7 @@ __global__ __launch_bounds__(kBlock) void ArgMaxRows(const float* __restrict__ a
         }
         start = n4 * 4;
     }
-    for (uint32_t i = start + threadIdx.x; i < p.kx; i += kBlock)
+    for (uint32_t i = start + threadIdx.x; i < p.kx; i += kThreads)
     {
         if (x[i] > value)
         {
@@ -594,7 +601,7 @@ __global__ __launch_bounds__(kBlock) void ArgMaxRows(const float* __restrict__ a
     {
         float v = bestValue[0];
         int32_t idx = bestIndex[0];
-        for (int w = 1; w < kWaves; ++w)
+        for (int w = 1; w < kThreads / kWave; ++w)
         {
             if (bestValue[w] > v || (bestValue[w] == v && bestIndex[w] < idx))
             {
@@ -701,6 +708,16 @@ extern "C" int muyo_argmax_f32(const LlamaGenericHeadPushConstants* pc, const fl
         return Fail(MUYO_E_DISPATCH, "%s: dispatch too large", name);
     }
     ArgMaxArgs p{pc->KX, pc->KY, dispatch_x, dispatch_y, dispatch_z};
-    hipLaunchKernelGGL(ArgMaxRows, dim3(static_cast<uint32_t>(slots)), dim3(kBlock), 0, AsStream(stream), a, d, p);
+    // Up to a workgroup per CU, rows of at least one batch of the large workgroup's loads (one row of
+    // 16384: 3.5 us small, 4.1 large; of 32768: 4.5 both; of 151936: 12.4 / 8.5 from L2; 128 rows of
+    // 151936: 27.3 / 16.4).
+    if (slots <= 256 && pc->KX >= 8 * 4 * 1024)
+    {
+        hipLaunchKernelGGL((ArgMaxRows<1024, 8>), dim3(static_cast<uint32_t>(slots)), dim3(1024), 0, AsStream(stream), a,
+                           d, p);
+        return LaunchStatus(name);
+    }
+    hipLaunchKernelGGL((ArgMaxRows<kBlock, 4>), dim3(static_cast<uint32_t>(slots)), dim3(kBlock), 0, AsStream(stream), a,
+                       d, p);
     return LaunchStatus(name);
 }

@@ -302,6 +302,41 @@ def test_argmax_ties_across_load_batches_and_tails(mh, gpu, orc, cols):
     assert np.array_equal(argmax(mh, gpu, x), want)
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 32768), (1, 151936), (256, 32771), (257, 32768), (3, 32767), (2, 36867)])
+def test_argmax_few_long_rows(mh, gpu, orc, rows, cols):
+    """Both workgroup shapes at the edges of the rule between them (256 rows, 32768 columns) and of
+    their load batches: ties, NaN and -inf (never the maximum; a row of nothing else gives 0), and
+    rows off 16-byte alignment."""
+    rng = np.random.default_rng(rows + cols)
+    x = rng.normal(0, 1, (rows, cols)).astype(np.float32)
+    want = np.argmax(x, axis=1)
+    assert np.array_equal(argmax(mh, gpu, x), want)
+    for row in range(rows):
+        kind = (row + cols) % 6
+        if kind == 0:
+            x[row, [cols - 1, 2048, 2047]] = 9.0       # the lowest of a tie
+            want[row] = 2047
+        elif kind == 1:
+            x[row, 0] = np.nan
+            x[row, 4000] = 7.0
+            want[row] = 4000
+        elif kind == 2:
+            x[row] = -np.inf
+            want[row] = 0
+        elif kind == 3:
+            x[row] = np.nan
+            x[row, cols - 2] = -3.0
+            want[row] = cols - 2
+        elif kind == 4:
+            x[row, [0, 1024]] = 11.0
+            want[row] = 0
+        else:
+            x[row] = np.nan
+            want[row] = 0
+    got = argmax(mh, gpu, x)
+    assert np.array_equal(got, want), (got, want)
+
+
 def test_argmax_batched_decode_shape(mh, gpu, orc):
     """4096 rows x 151936 logits N(0, 2): 256 rows against the oracle, all rows against torch.argmax."""
     torch = gpu
