@@ -160,7 +160,10 @@ struct SwiGluEpi
 /// every wave's part of the slab has arrived and every wave is done with the buffer that the next
 /// loads overwrite. Rows are not padded (the load writes 1 KB at a stretch), so each row's 16-byte
 /// chunks are permuted by the row number instead, on the global side of the load; the fragment
-/// reads of eight consecutive rows then touch every bank once.
+/// reads of eight consecutive rows then touch no bank twice. (The 16 that share the 64 banks still
+/// meet in pairs. A permutation without that, 4.0 conflict cycles per LDS instruction cycle less,
+/// left the GEMMs within 0.4 % and whole prompts of 613 rows 2 % slower by its address
+/// instructions: waves wait on LDS 2 to 6 % of their cycles.)
 ///
 /// The compiler does not see these loads: it neither counts them nor orders LDS reads after
 /// them. WaitAndMeet counts them (a wave's loads complete in order, kLoads a slab).
