@@ -347,6 +347,12 @@ __global__ __launch_bounds__(256) void RopeSplitAppendKernel(const float* __rest
 /// stores and the same arithmetic per element (head_dim % 8 == 0, buffers aligned). The table of
 /// powers is requested before the partial sums, so the angles are computed while the sums are
 /// in flight (loads complete in order).
+///
+/// kParts is the most K splits summed, all requested before the first is added; 1 means whole sums
+/// (bias included) in qkv. The parts' registers cost waves in flight: whole sums of 28 / 4 heads of
+/// 128, 1024 rows, 7.0 us through the eight-part kernel (108 registers, four waves per SIMD), 6.2
+/// through the one-part kernel (44, eight); 2048 rows 12.5 / 12.0.
+template <uint32_t kParts>
 __global__ __launch_bounds__(256) void RopeSplitAppendQuadKernel(const float* __restrict__ qkv, uint32_t rows,
                                                                  int32_t pos0, uint32_t heads, uint32_t kvHeads,
                                                                  uint32_t headDim, uint32_t maxSeq,
@@ -371,19 +377,18 @@ __global__ __launch_bounds__(256) void RopeSplitAppendQuadKernel(const float* __
     const uint32_t width = (heads + 2 * kvHeads) * headDim;
     const float* row = qkv + static_cast<uint64_t>(m) * width;
     const uint64_t stride = static_cast<uint64_t>(rows) * width;
-    // Every split's part of four columns, requested before the first is added.
     struct Parts
     {
-        float4v v[kMaxGemmSplits];
+        float4v v[kParts];
         float4v bias;
     };
     auto request = [&](uint32_t col) {
         Parts p;
         p.v[0] = *reinterpret_cast<const float4v*>(row + col);
-        if (splits > 1)
+        if constexpr (kParts > 1)
         {
 #pragma unroll
-            for (uint32_t z = 1; z < kMaxGemmSplits; ++z)
+            for (uint32_t z = 1; z < kParts; ++z)
             {
                 if (z < splits)
                 {
@@ -396,10 +401,10 @@ __global__ __launch_bounds__(256) void RopeSplitAppendQuadKernel(const float* __
     };
     auto total = [&](const Parts& p) {
         float4v a = p.v[0];
-        if (splits > 1)
+        if constexpr (kParts > 1)
         {
 #pragma unroll
-            for (uint32_t z = 1; z < kMaxGemmSplits; ++z)
+            for (uint32_t z = 1; z < kParts; ++z)
             {
                 if (z < splits)
                 {
@@ -525,8 +530,11 @@ hipError_t LaunchRopeSplitAppend(hipStream_t s, const float* qkv, uint32_t rows,
     {
         // Threads: four pairs of a rotated head each, or four v channels.
         const uint64_t quads = static_cast<uint64_t>(rows) * ((heads + kvHeads) * (headDim / 8) + kvHeads * headDim / 4);
-        hipLaunchKernelGGL(RopeSplitAppendQuadKernel, dim3(CeilDiv(quads, 256)), dim3(256), 0, s, qkv, rows, pos0,
-                           heads, kvHeads, headDim, maxSeq, ropePow, qhi, qlo, kcache, vcache, splits, bias);
+        const auto kernel = splits == 1   ? RopeSplitAppendQuadKernel<1>
+                            : splits <= 4 ? RopeSplitAppendQuadKernel<4>
+                                          : RopeSplitAppendQuadKernel<kMaxGemmSplits>;
+        hipLaunchKernelGGL(kernel, dim3(CeilDiv(quads, 256)), dim3(256), 0, s, qkv, rows, pos0, heads, kvHeads,
+                           headDim, maxSeq, ropePow, qhi, qlo, kcache, vcache, splits, bias);
         return hipGetLastError();
     }
     hipLaunchKernelGGL(RopeSplitAppendKernel, dim3(CeilDiv(total, 256)), dim3(256), 0, s, qkv, rows, pos0, heads,
