@@ -538,7 +538,9 @@ struct AttnPlan
 /// end, or the longest one alone; with chunks, the partials' way to memory and back and the merge.
 /// A CU takes 2.2 us per step of a workgroup (head_dim 64: 1.5), whether it holds one or two. Over
 /// 17 measured launches (20 to 2048 rows at cache rows 0 to 5000, both head sizes) the choice was
-/// within 8 % of the fastest.
+/// within 8 % of the fastest. The merge of a few rows at head_dim 64 costs less (32 rows at cache row
+/// 100, 14 / 2 heads, three steps in one chunk 9.6 us, in three 8.5; 250 rows at row 0, four steps,
+/// 10.8 / 10.0).
 ///
 /// At head_dim 128, whose sums run over a whole chunk (kStepSums), a chunk is at most twice an
 /// eighth of the range or 1024 keys: the error against 64 bits stays that of eighths and 512 keys
@@ -567,7 +569,9 @@ AttnPlan PlanAttention(uint32_t rows, int32_t pos0, uint32_t heads, uint32_t kvH
         double us = std::max(all + one / 2.0, one + 3.0);
         if (chunks > 1)
         {
-            us += 4.0 + 2.0 * (range / chunkTiles) * rows * heads * (headDim + 2) * 4.0 / 5.0e6;
+            // (A small merge follows at once; one of a megabyte or more starts with its own loads.)
+            const double partialsUs = (range / chunkTiles) * rows * heads * (headDim + 2) * 4.0 / 5.0e6;
+            us += 2.0 * partialsUs + (headDim == 128 ? 4.0 : 2.35 + std::min(2.75 * partialsUs, 1.65));
         }
         if (us < bestUs)
         {

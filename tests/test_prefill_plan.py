@@ -39,3 +39,9 @@ def test_attention_chunks_cover_the_keys(attention_plan, shape):
 def test_attention_of_three_key_tiles_is_one_chunk(attention_plan, shape, rows, pos0):
     """A merge costs more than a second 64-key step, also where the range is an odd number of tiles."""
     assert attention_plan(*shape, rows, pos0) == (1, 4)
+
+
+@pytest.mark.parametrize("rows,pos0,chunks", [(32, 100, 3), (45, 100, 3), (130, 0, 1), (250, 0, 4), (301, 100, 7)])
+def test_attention_chunks_of_small_merges(attention_plan, rows, pos0, chunks):
+    """14 / 2 heads of 64: three steps or more are split where the merge is small."""
+    assert attention_plan(14, 2, 64, rows, pos0)[0] == chunks
