@@ -157,7 +157,12 @@ __device__ constexpr int KeyOf(int r) { return 32 * (r / 16) + 8 * (r % 16 / 4) 
 /// covers keys [c * C, (c + 1) * C), C = 32 * chunkTiles; a query tile with more keys than C leaves
 /// each chunk's unnormalised softmax partial (running max, sum, P.V) in slot c of `part` for
 /// PrefillAttnMergeKernel, one with at most C writes its planes directly.
-template <int kHd>
+///
+/// kKeys keys (32 or 64) of a step are handled at a time. At head_dim 128 the scores and weights of
+/// 64 would not fit the registers beside q and o. At 64 they do, and a wave meets half as many
+/// phases; but a range that ends in the first half of a step then pays for the other half
+/// (kShortTiles).
+template <int kHd, int kKeys>
 __global__ __launch_bounds__(kWave* kAttnWaves, 2) void PrefillAttentionKernel(
     const uint16_t* __restrict__ qhi, const uint16_t* __restrict__ qlo, const uint16_t* __restrict__ kcache,
     const uint16_t* __restrict__ vcache, uint16_t* __restrict__ ohi, uint16_t* __restrict__ olo, uint32_t rows,
@@ -166,9 +171,6 @@ __global__ __launch_bounds__(kWave* kAttnWaves, 2) void PrefillAttentionKernel(
 {
     constexpr int kWaves = kAttnWaves;
     constexpr int kStages = kHd == 128 ? 2 : 3;
-    // Keys handled at a time: at head_dim 128 the scores and weights of 64 would not fit the
-    // registers beside q and o.
-    constexpr int kKeys = kHd == 128 ? 32 : 64;
     // A step's products summed by themselves and added to the rescaled total: one rounding at the
     // total's size per 64 keys instead of eight, where the registers allow.
     constexpr bool kStepSums = kHd == 64;
@@ -581,6 +583,16 @@ AttnPlan PlanAttention(uint32_t rows, int32_t pos0, uint32_t heads, uint32_t kvH
     }
     return best;
 }
+/// At head_dim 64, ranges of up to this many tiles of 32 keys are handled 32 keys at a time. 14 / 2
+/// heads, us, 64 keys / 32: one row at cache row 0 4.8 / 4.0, 32 rows 6.3 / 5.4, 64 rows 6.3 / 6.2.
+/// (Up to six tiles 32 keys are as fast or faster, 80 rows 6.8 / 6.3; but the sums meet the total
+/// twice as often, and one row after 100 is 2.1e-7 / 2.5e-7 off its 64-bit value.)
+constexpr uint32_t kShortTiles = 2;
+
+uint32_t KeysAtATime(uint32_t rows, int32_t pos0, uint32_t headDim)
+{
+    return headDim == 64 && AttnKeyTiles(CeilDiv(rows, 32) - 1, rows, pos0) > kShortTiles ? 64 : 32;
+}
 }  // namespace
 
 hipError_t LaunchPrefillAttention(hipStream_t s, const uint16_t* qhi, const uint16_t* qlo, const uint16_t* kcache,
@@ -604,9 +616,11 @@ hipError_t LaunchPrefillAttention(hipStream_t s, const uint16_t* qhi, const uint
     }
     const uint32_t pairs = CeilDiv(rows, 32) * (heads / kvHeads);
     const dim3 grid(CeilDiv(pairs, kAttnWaves) * plan.chunks * kvHeads);
-    hipLaunchKernelGGL((headDim == 128 ? PrefillAttentionKernel<128> : PrefillAttentionKernel<64>), grid,
-                       dim3(kWave * kAttnWaves), 0, s, qhi, qlo, kcache, vcache, ohi, olo, rows, pos0, heads, kvHeads,
-                       maxSeq, scale, plan.chunkTiles, part);
+    const auto kernel = headDim == 128                          ? PrefillAttentionKernel<128, 32>
+                        : KeysAtATime(rows, pos0, headDim) == 32 ? PrefillAttentionKernel<64, 32>
+                                                                 : PrefillAttentionKernel<64, 64>;
+    hipLaunchKernelGGL(kernel, grid, dim3(kWave * kAttnWaves), 0, s, qhi, qlo, kcache, vcache, ohi, olo, rows, pos0,
+                       heads, kvHeads, maxSeq, scale, plan.chunkTiles, part);
     if (plan.chunks > 1)
     {
         const uint64_t threads = static_cast<uint64_t>(rows) * heads * (headDim / 4);
@@ -617,11 +631,13 @@ hipError_t LaunchPrefillAttention(hipStream_t s, const uint16_t* qhi, const uint
 }
 }  // namespace muyo
 
-// For the tests (no device needed): the chunks of a launch and their length in tiles of 32 keys.
+// For the tests (no device needed): the chunks of a launch, their length in tiles of 32 keys, and the
+// keys handled at a time.
 extern "C" void muyo_prefill_attention_plan(uint32_t rows, int32_t pos0, uint32_t heads, uint32_t kvHeads,
-                                            uint32_t headDim, uint32_t workspace, uint32_t plan[2])
+                                            uint32_t headDim, uint32_t workspace, uint32_t plan[3])
 {
     const muyo::AttnPlan p = muyo::PlanAttention(rows, pos0, heads, kvHeads, headDim, workspace != 0);
     plan[0] = p.chunks;
     plan[1] = p.chunkTiles;
+    plan[2] = muyo::KeysAtATime(rows, pos0, headDim);
 }

@@ -462,6 +462,22 @@ def test_prefill_attention_edges_against_float64(mh, gpu, heads, kv_heads, head_
     assert float((got - want).norm() / want.norm()) <= 2e-6 + top * 2.0 ** -22
 
 
+@pytest.mark.parametrize("heads,kv_heads,rows,pos0,max_seq,spread", [
+    (6, 3, 1, 0, 1, 1.0),       # one key
+    (4, 4, 32, 0, 33, 30.0),    # one whole tile of keys, maxima that rise past the 2^8 slack
+    (4, 4, 33, 31, 64, 1.0),    # two tiles to the last key
+    (14, 2, 64, 0, 64, 1.0),    # two tiles: the last range of 32 keys at a time
+    (12, 4, 20, 44, 64, 30.0),
+    (14, 2, 65, 0, 70, 1.0),    # one key past it
+])
+@pytest.mark.parametrize("workspace", [False, True])
+def test_prefill_attention_short_ranges_against_float64(mh, gpu, heads, kv_heads, rows, pos0, max_seq, spread,
+                                                        workspace):
+    """head_dim 64 on both sides of the step from 32 keys at a time to 64."""
+    test_prefill_attention_edges_against_float64(mh, gpu, heads, kv_heads, 64, rows, pos0, max_seq, 0.125, spread,
+                                                 workspace)
+
+
 def test_prefill_attention_refusals(mh, gpu):
     lib = mh.load()
     fake = ctypes.c_void_p(256)
