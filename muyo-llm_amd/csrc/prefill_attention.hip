@@ -233,8 +233,8 @@ __global__ __launch_bounds__(kWave* kAttnWaves, 2) void PrefillAttentionKernel(
         const uint32_t row0 = min(keyBegin + step * kAttnStep + g * kRowsPerLoad, maxSeq - 1);
         const uint16_t* base = (isV ? vcache : kcache) + cacheBase + static_cast<uint64_t>(row0) * kHd;
         const uint32_t offset = min(laneRow, maxSeq - 1 - row0) * kRowBytes + (isV ? vLoadAt : kAt);
-        const uint32_t to = ldsBase + (stage * 2 + isV) * kMatrixBytes + g * 1024;
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(offset), "s"(base));
+        LoadToLds(ldsBase + stage * 2 * kMatrixBytes + wave * 1024,
+                  isV * kMatrixBytes + i % kMatrixLoads * kWaves * 1024, offset, base);
     };
 
     // Scores are scaled by |scale| (in log2 units) inside the exponential, so that the running

@@ -39,6 +39,29 @@ __device__ __forceinline__ void StoreSplit4(uint16_t* hi, uint16_t* lo, uint64_t
     *reinterpret_cast<half4*>(hi + at) = h;
     *reinterpret_cast<half4*>(lo + at) = l;
 }
+
+/// Requests 16 bytes per lane from base + offset bytes (base uniform across the wave) straight into
+/// LDS: the wave's 64 pieces land in lane order in the 1 KB at LDS address to + more (`more` a
+/// constant once the loops around are unrolled). The compiler does not see the load: it neither
+/// counts it nor orders LDS reads after it (WaitAndMeet does), and keeps no wait states before it.
+/// It needs one after m0 is written, and would need five after a vector instruction has written
+/// its scalar base (v_readfirstlane, the return of a spilled scalar): the base goes through a
+/// scalar move, which waits for either by itself and is the wait state of m0. (m0 is a register
+/// in which the compiler keeps nothing across instructions.)
+///
+/// A wave issues a slab's loads one instruction at a time, so these count in a GEMM of few rows,
+/// us, 17 rows of 4864 x 896: 24.3 with the LDS address added up before and an s_nop for m0's wait
+/// state alone, 26.1 with an s_nop for the base's five, 24.8 with the move, 21.1 with the move and
+/// the addition into m0.
+__device__ __forceinline__ void LoadToLds(uint32_t to, uint32_t more, uint32_t offset, const void* base)
+{
+    uint64_t scalarBase;
+    asm volatile("s_add_u32 m0, %1, %2\n\ts_mov_b64 %0, %4\n\tglobal_load_lds_dwordx4 %3, %0"
+                 : "=&s"(scalarBase)
+                 : "s"(to), "i"(more), "v"(offset), "s"(base)
+                 : "scc");
+}
+
 /// Waits until at most kLeft of this wave's loads are in flight and its LDS reads are done, then
 /// meets the other waves.
 template <int kLeft>

@@ -155,18 +155,15 @@ struct SwiGluEpi
 /// of 16 columns, their sums meeting in LDS at the end.
 ///
 /// K advances kBk columns at a time through kStages LDS buffers. The loads go from memory to LDS
-/// without passing through registers (global_load_lds_dwordx4: a wave's 64 x 16 bytes land in 1 KB
-/// of LDS in lane order), up to kStages - 1 slabs ahead, and a slab costs one barrier: past it,
-/// every wave's part of the slab has arrived and every wave is done with the buffer that the next
-/// loads overwrite. Rows are not padded (the load writes 1 KB at a stretch), so each row's 16-byte
+/// without passing through registers (LoadToLds), up to kStages - 1 slabs ahead, and a slab costs
+/// one barrier: past it, every wave's part of the slab has arrived and every wave is done with the
+/// buffer that the next loads overwrite. WaitAndMeet counts the loads (a wave's complete in order,
+/// kLoads a slab). Rows are not padded (the load writes 1 KB at a stretch), so each row's 16-byte
 /// chunks are permuted by the row number instead, on the global side of the load; the fragment
 /// reads of eight consecutive rows then touch no bank twice. (The 16 that share the 64 banks still
 /// meet in pairs. A permutation without that, 4.0 conflict cycles per LDS instruction cycle less,
 /// left the GEMMs within 0.4 % and whole prompts of 613 rows 2 % slower by its address
 /// instructions: waves wait on LDS 2 to 6 % of their cycles.)
-///
-/// The compiler does not see these loads: it neither counts them nor orders LDS reads after
-/// them. WaitAndMeet counts them (a wave's loads complete in order, kLoads a slab).
 ///
 /// What bounds it. With random data the matrix cores alone sustain 1.67 PFLOP/s on this part (its
 /// power limit; 2.3 with zeros), and 1.5 with an LDS fragment read for every two operations. Loads
@@ -192,7 +189,7 @@ struct GemmTile
     static constexpr int kChunks = kBk / 8;               // 16-byte chunks per row
     static constexpr int kRowsPerLoad = kWave / kChunks;  // rows one load instruction brings
     static constexpr int kGroups = kRows / kRowsPerLoad;
-    static constexpr int kLoads = (kGroups + kWaves - 1) / kWaves;  // per wave and slab
+    static constexpr int kLoads = kGroups / kWaves;       // per wave and slab
     static constexpr int kStageBytes = kRows * kRowBytes;
     static constexpr int kSteps = kBk / 16 / kWk;         // per wave and slab
     static constexpr int kMinWaves = (kWaves * kPerCu + 3) / 4;  // per SIMD
@@ -200,6 +197,7 @@ struct GemmTile
     static constexpr bool kLowSums = kMb * kNb <= 4;      // two sums per block
     static constexpr int kSumFloats = 1024 * kNb * kMb;   // a wave's tile
     static_assert(kRows % kRowsPerLoad == 0 && kBm % kRowsPerLoad == 0 && 16 % kRowsPerLoad == 0, "row groups");
+    static_assert(kGroups % kWaves == 0, "every wave has as many loads in flight as WaitAndMeet counts");
     static_assert(kBk % (16 * kWk) == 0 && kGemmSplitUnit % kBk == 0, "steps");
     static_assert(kStages >= 2 && kStages <= 5 && kStages * kStageBytes * kPerCu <= 160 * 1024, "LDS");
     static_assert((kWk - 1) * kWm * kWn * kSumFloats * 4 <= kStages * kStageBytes, "LDS of the K sums");
@@ -250,14 +248,13 @@ __global__ __launch_bounds__(T::kThreads, T::kMinWaves) void GemmSplitKernel(con
     // group's, uniform across the wave, plus the lane's offset. A lane whose row lies past the
     // matrix reads the group's first row (clamped to the last) instead, and one whose chunk lies
     // past kEnd the row's first chunk of the slab: in bounds, and either not stored or zeroed
-    // below. A wave with fewer groups than kLoads brings its last one again, so that the counts
-    // of WaitAndMeet hold for every wave.
+    // below.
     const uint32_t groupRow = lane / T::kChunks;
     const uint32_t ldsBase =
         static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)lds));
     auto load = [&](uint32_t stage, uint32_t k0, int i)
     {
-        const uint32_t g = min(wave + i * T::kWaves, static_cast<uint32_t>(T::kGroups) - 1);
+        const uint32_t g = wave + i * T::kWaves;
         const uint32_t r = g * T::kRowsPerLoad;
         const uint32_t row = r + groupRow;
         const uint32_t chunk = (lane % T::kChunks) ^ (kBk == 32 ? (row >> 1) & 3u : row & 7u);
@@ -278,8 +275,7 @@ __global__ __launch_bounds__(T::kThreads, T::kMinWaves) void GemmSplitKernel(con
             live = epi.Live(u, groupRow);
         }
         const uint32_t offset = live ? first + groupRow * k * 2 : first;
-        const uint32_t to = ldsBase + stage * T::kStageBytes + g * 1024;
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(offset), "s"(base));
+        LoadToLds(ldsBase + stage * T::kStageBytes + wave * 1024, i * T::kWaves * 1024, offset, base);
     };
 
     const uint32_t kg = wave / (kWm * kWn);
