@@ -108,11 +108,11 @@ def test_rms_norm_split_matches_oracle(mh, gpu, orc):
 GEMM_SHAPES = [
     (1, 8, 8),          # one token, one 16-byte chunk of K
     (37, 100, 72),      # ragged rows, n not a multiple of 32, k not of 64
-    (128, 128, 64),     # exactly one 128 x 128 tile
+    (128, 128, 64),     # whole tiles
     (200, 1152, 896),   # 0.5B QKV
     (300, 896, 896),    # 0.5B o_proj
     (67, 896, 4864),    # 0.5B down: long K
-    (640, 1152, 896),   # 45 tiles of 128 x 128: the 64-token tiles
+    (640, 1152, 896),   # 0.5B QKV over more rows than K splits of eight are for
 ]
 
 
@@ -167,9 +167,9 @@ def test_gemm_split_integer_inputs_are_exact(mh, gpu):
 
 @pytest.mark.parametrize("rows,n,k", [(1990, 4600, 136), (1990, 16300, 72)])
 def test_gemm_split_large_grids_integer_exact(mh, gpu, rows, n, k):
-    """Integer inputs on the 128 x 128 and 128 x 256 tile kernels (576 and 1040 tiles, the second
-    with token tiles fastest): a last token tile of 70 rows, a last weight tile of 120 or 172
-    rows and a K tail inside the last K tile, whose lanes past the matrix read in-bounds rows."""
+    """Integer inputs over grids of several rounds of workgroups: a ragged last token tile, a ragged last
+    weight tile, several groups of token tiles, and a K tail inside the last slab, whose lanes past
+    the matrix read in-bounds rows."""
     torch = gpu
     rng = np.random.default_rng(rows + n + k)
     a = rng.integers(-8, 9, (rows, k)).astype(np.float32)
@@ -183,7 +183,7 @@ def test_gemm_split_large_grids_integer_exact(mh, gpu, rows, n, k):
 
 
 def test_gemm_swiglu_wide_tiles_integer_products(mh, gpu):
-    """The 128 x 256 swiglu tiles (1040 of them) on integer inputs: both products exact, the
+    """The swiglu GEMM over several rounds of workgroups on integer inputs: both products exact, the
     swiglu of them to the planes' precision; ragged token and ffn tiles and a K tail."""
     torch = gpu
     rows, ffn, k = 1990, 8200, 40
@@ -238,8 +238,8 @@ TILE_SHAPES = [
 @pytest.mark.parametrize("rows,n,k", TILE_SHAPES)
 def test_gemm_tile_shapes_exact_with_both_planes(mh, gpu, rows, n, k):
     """Values whose products and sums are exact in f32 (hi and weights integers up to 2, lo a
-    multiple of 2^-10: at most 11 + 1 + 10 bits), so the plain GEMM must match to the bit and the
-    swiglu GEMM to the planes' precision."""
+    multiple of 2^-11 up to 2^-10: sums below 2^12 in steps of 2^-11, 23 bits), so the plain GEMM must
+    match to the bit and the swiglu GEMM to the planes' precision."""
     torch = gpu
     g = torch.Generator(device="cuda").manual_seed(rows * 31 + n + k)
 
@@ -364,9 +364,8 @@ def test_prefill_attention_matches_per_token_attention(mh, gpu, orc, heads, kv_h
 
 @pytest.mark.parametrize("heads,kv_heads,head_dim", [(14, 2, 64), (28, 4, 128)])
 def test_prefill_attention_full_prompt(mh, gpu, orc, heads, kv_heads, head_dim):
-    """2048 queries: the 0.5B shape's groups of 7 split over two workgroups per tile, the 7B shape's
-    whole groups (its grid alone fills the chip); rows checked at tile edges and spread over the
-    prompt."""
+    """2048 queries without a workspace: one chunk of 64 key tiles; rows checked at tile edges and spread
+    over the prompt."""
     rows = 2048
     check = [0, 1, 31, 32, 33, 500, 1023, 1024, 1537, 2015, 2016, 2046, 2047]
     prefill_attention_case(mh, gpu, orc, heads, kv_heads, head_dim, rows, 0, rows, 7 + heads, check)
@@ -384,19 +383,28 @@ def test_prefill_attention_ignores_rows_past_the_prompt(mh, gpu, orc, heads, kv_
     prefill_attention_case(mh, gpu, orc, heads, kv_heads, head_dim, rows, pos0, max_seq, 3 + rows, poison=True)
 
 
-@pytest.mark.parametrize("heads,kv_heads,head_dim,rows,pos0,max_seq,check", [
-    (14, 2, 64, 512, 0, 512, None),         # last tile exactly 16 key tiles: nothing split
-    (14, 2, 64, 513, 0, 544, None),         # one query past it: a 16 + 1 split of the last tile
-    (14, 2, 64, 600, 0, 640, None),         # tiles 16..18 in two chunks
-    (14, 2, 64, 40, 1000, 2048, None),      # after an earlier prompt: every tile split in three
-    (28, 4, 128, 33, 2015, 2048, None),     # 7B heads, ending at the last cache row: four chunks
-    (8, 1, 128, 64, 1100, 1200, None),      # a full group of 8 over a ragged cache
-    (4, 4, 64, 96, 8000, 8192, range(0, 96, 5)),  # 251+ key tiles: chunks of 32 key tiles, eight per tile
-    (14, 2, 64, 2048, 0, 2048, [0, 31, 511, 512, 543, 544, 1000, 1535, 1536, 2046, 2047]),
-    (28, 4, 128, 2048, 0, 2048, [0, 33, 512, 1023, 1024, 1500, 2015, 2016, 2047]),
-    (14, 2, 64, 2100, 0, 2112, [0, 2047, 2048, 2099]),  # past the decoder's 2048-row passes: 170 items
-    (14, 2, 64, 4160, 0, 4160, [0, 2047, 3000, 4159]),  # its chunks would be 564 work items: runs unsplit
-])
+# With a workspace: shape, rows, first position, cache rows, the queries checked, and what the launch
+# is planned as (chunks, tiles of 32 keys a chunk; test_prefill_plan.py holds the plans to it). In a
+# prompt from row 0 the query tiles of up to a chunk's key tiles write their planes, the next one
+# leaves two partials, the second of one tile.
+CHUNK_CASES = [
+    (14, 2, 64, 512, 0, 512, None, (4, 4)),         # 16 key tiles: four whole chunks
+    (14, 2, 64, 513, 0, 544, None, (5, 4)),         # one query past them: a fifth chunk of one tile
+    (14, 2, 64, 600, 0, 640, None, (5, 4)),
+    (14, 2, 64, 129, 0, 160, None, (1, 6)),         # one chunk, with the workspace unused
+    (14, 2, 64, 40, 1000, 2048, None, (6, 6)),      # after an earlier prompt: every tile split
+    (28, 4, 128, 33, 2015, 2048, None, (8, 8)),     # 7B heads, ending at the last cache row: every chunk
+    (28, 4, 128, 300, 0, 300, range(0, 300, 7), (3, 4)),
+    (8, 1, 128, 64, 1100, 1200, None, (7, 6)),      # a full group of 8 over a ragged cache
+    (4, 4, 64, 96, 8000, 8192, range(0, 96, 5), (8, 32)),  # 251+ key tiles: long chunks, the last one short
+    (14, 2, 64, 2048, 0, 2048, [0, 31, 511, 512, 543, 544, 1000, 1535, 1536, 2046, 2047], (4, 16)),
+    (28, 4, 128, 2048, 0, 2048, [0, 33, 512, 1023, 1024, 1500, 2015, 2016, 2047], (2, 32)),
+    (14, 2, 64, 2100, 0, 2112, [0, 575, 576, 2047, 2048, 2099], (4, 18)),  # past the decoder's 2048-row passes
+    (14, 2, 64, 4160, 0, 4160, [0, 1087, 1088, 2047, 3000, 4159], (4, 34)),
+]
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim,rows,pos0,max_seq,check", [case[:7] for case in CHUNK_CASES])
 def test_prefill_attention_key_chunks_match_per_token_attention(mh, gpu, orc, heads, kv_heads, head_dim, rows, pos0,
                                                                max_seq, check):
     """Query tiles split into key chunks, combined by the merge kernel, against the oracle's
@@ -406,7 +414,7 @@ def test_prefill_attention_key_chunks_match_per_token_attention(mh, gpu, orc, he
 
 
 @pytest.mark.parametrize("heads,kv_heads,head_dim,rows,pos0,max_seq", [
-    (14, 2, 64, 600, 30, 1024),     # the split tiles' last key tile mostly past the prompt
+    (14, 2, 64, 600, 30, 1024),     # the split tiles' last key tile ends past the prompt
     (28, 4, 128, 40, 1000, 2048),
 ])
 def test_prefill_attention_key_chunks_ignore_rows_past_the_prompt(mh, gpu, orc, heads, kv_heads, head_dim, rows,
@@ -561,7 +569,7 @@ def test_decoder_prefill_odd_shapes(mh, gpu, orc, name):
 
 def test_decoder_prefill_after_long_cache(mh, gpu, orc):
     """A 100-token prompt appended at cache row 15000 of 16384 (o_proj per kv group at head_dim
-    128): each query tile's 470-472 key tiles split into eight chunks and merged."""
+    128): each query tile's 470-472 key tiles in eight chunks of up to 60 and merged."""
     shape = dict(layers=1, hidden=512, ffn=512, heads=12, kv_heads=4, head_dim=128, vocab=300, max_seq=16384)
     dec, model = make_pair(mh, orc, shape, seed=53, kv_positions=15000, kv_seed=54)
     with dec:
@@ -616,9 +624,8 @@ def test_decoder_prefill_equals_steps_on_gpu(mh, gpu, orc):
 
 @pytest.mark.parametrize("count", [2048, 1990])
 def test_decoder_prefill_7b_width_full_prompt_equals_steps(mh, gpu, orc, count):
-    """The 7B widths over a 2048-token (and a 1990-token: ragged last token tiles) prompt, where
-    q|k|v takes 128 x 128 tiles over two K halves, o_proj and down 128 x 256 tiles over two K
-    halves and the gate+up 128 x 256 tiles: the same logits, cache rows and next token as the
+    """The 7B widths over a 2048-token (and a 1990-token: ragged last token tiles) prompt, whose GEMMs take
+    the largest tiles, some over K splits: the same logits, cache rows and next token as the
     decoder's own steps."""
     shape = dict(mh.QWEN25_7B, layers=2)
     tokens = prompt(orc, count, shape["vocab"], 63)
@@ -641,7 +648,7 @@ def test_decoder_prefill_7b_width_full_prompt_equals_steps(mh, gpu, orc, count):
 @pytest.mark.timeout(900)
 def test_decoder_prefill_7b_width_1024_tokens_matches_oracle(mh, gpu, orc):
     """The 7B widths (hidden 3584, ffn 18944, 28/4 heads of 128) over a 1024-token prompt from row
-    0, which takes the 128 x 256 gate+up tiles, against the oracle fed token by token: the last
+    0 against the oracle fed token by token: the last
     position's logits, the next token and every cache row (a small vocabulary keeps the oracle's
     LM head cheap; the projections are full width)."""
     orc.set_threads(16)

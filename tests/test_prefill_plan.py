@@ -4,6 +4,8 @@ import ctypes
 
 import pytest
 
+from test_prefill_gpu import CHUNK_CASES
+
 
 @pytest.fixture(scope="module")
 def attention_plan(mh):
@@ -53,3 +55,9 @@ def test_attention_of_short_ranges_takes_32_keys_at_a_time(attention_plan):
 def test_attention_chunks_of_small_merges(attention_plan, rows, pos0, chunks):
     """14 / 2 heads of 64: three steps or more are split where the merge is small."""
     assert attention_plan(14, 2, 64, rows, pos0)[0] == chunks
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim,rows,pos0,max_seq,check,planned", CHUNK_CASES)
+def test_attention_chunk_cases_are_planned_as_they_say(attention_plan, heads, kv_heads, head_dim, rows, pos0, max_seq,
+                                                       check, planned):
+    assert attention_plan(heads, kv_heads, head_dim, rows, pos0)[:2] == planned
