@@ -167,16 +167,14 @@ struct SwiGluEpi
 ///
 /// What bounds it. With random data the matrix cores alone sustain 1.67 PFLOP/s on this part (its
 /// power limit; 2.3 with zeros), and 1.5 with an LDS fragment read for every two operations. Loads
-/// from L2 run at 34 TB/s but anything past it at 7, so a tile order that lets every XCD fetch
-/// every weight row is bound by that: workgroups are dealt to the XCDs round-robin, and XCD x
-/// takes the x-th eighth of the tiles instead (GemmOrder), 3.3 MB of each XCD's own rather than
-/// all 17 MB of the 0.5B gate+up weight. A single wave per SIMD leaves the matrix cores idle
-/// between a barrier and its first fragments: the shapes have two (or two workgroups per CU) where
-/// LDS allows.
-/// Measured, before (a register-staged kernel, one LDS buffer) and now, us: 0.5B gate+up
-/// 301 rows 29.5 / 18.4, 613 rows 36.7 / 29.9; down 301 rows 82 / 24; 613 rows over K splits
-/// 34 / 22.5; q|k|v 613 rows 12.5 / 8.7; 7B gate+up 45 rows 91 / 55, 2048 rows 999 / 936; down
-/// 45 rows 78 / 36, 2048 rows 494 / 467.
+/// from L2 run at 34 TB/s but anything past it at 7, so what every XCD has to fetch counts
+/// (GemmOrder). A single wave per SIMD leaves the matrix cores idle between a barrier and its first
+/// fragments: the shapes have two (or two workgroups per CU) where LDS allows.
+/// Measured at the unsplit entry points, before (a register-staged kernel, one LDS buffer) and now,
+/// us: 0.5B gate+up 301 rows 29 / 18.0, 613 rows 41 / 30.4, 2048 rows 94 / 94; down 301 rows
+/// 82 / 22.4, 2048 rows 85 / 51; q|k|v 613 rows 21 / 10.0; 7B gate+up 45 rows 99 / 65, 2048 rows
+/// 1054 / 990; down 45 rows 308 / 84, 2048 rows 621 / 549; o_proj 2048 rows 123 / 111; q|k|v
+/// 2048 rows 194 / 156.
 template <int kWm, int kWn, int kWk, int kMb, int kNb, int kStages, int kBk, int kPerCu>
 struct GemmTile
 {
@@ -204,14 +202,19 @@ struct GemmTile
 };
 
 /// This workgroup's tile and K split. Workgroups are dealt to the 8 XCDs round-robin by id; with
-/// the renumbering XCD x runs a contiguous run of the sequence (split, then weight tiles, then
-/// token tiles fastest, or the last two swapped), so its L2 holds its own share of the slower
-/// dimension. Which dimension is the slower one: the larger operand's, read once over the chip
-/// while the other is read by every XCD. (The results do not depend on where a workgroup runs.)
+/// the renumbering XCD x runs the x-th eighth of one sequence: the splits, in each the groups of
+/// `group` token tiles, in each the weight tiles, in each the group's token tiles. (The results do
+/// not depend on where a workgroup runs.)
+///
+/// What an XCD's resident workgroups read of a slab comes from past its L2 once: the rows of the
+/// group's token tiles and of the weight tiles beside them, the fewest when the two are about as
+/// many (GroupTiles has the rule). With all token tiles in a group instead (or all weight tiles, where the
+/// activations were the larger operand), 8192 rows of 14336 x 4096 gate+up took 3.92 ms, with groups
+/// of four 256-row tiles 3.14; 2048 rows of 4864 x 896 on 128 x 256 tiles 95.4 / 93.1 us, 8192 rows
+/// of 3584 x 3584 383 / 350.
 struct GemmOrder
 {
-    uint32_t mTiles, nTiles;
-    bool mFast;
+    uint32_t mTiles, nTiles, group;
 
     __device__ void Tile(uint32_t& mt, uint32_t& nt, uint32_t& z) const
     {
@@ -220,8 +223,10 @@ struct GemmOrder
         const uint32_t plane = mTiles * nTiles;
         z = id / plane;
         const uint32_t t = id % plane;
-        mt = mFast ? t % mTiles : t / nTiles;
-        nt = mFast ? t / mTiles : t % nTiles;
+        const uint32_t first = t / (group * nTiles) * group;
+        const uint32_t width = min(group, mTiles - first);
+        mt = first + t % (group * nTiles) % width;
+        nt = t % (group * nTiles) / width;
     }
 };
 
@@ -481,31 +486,34 @@ __global__ __launch_bounds__(T::kThreads, T::kMinWaves) void GemmSplitKernel(con
 }
 
 /// The tile shapes, X(index, waves m, n, k, blocks m, n, LDS stages, K slab, workgroups per CU).
-/// Seven of eighteen that were measured over the prefill's GEMMs (both models' four matrices, 7 to
-/// 2048 rows, every K split): with these seven the best choice per GEMM is within 1 % of the best
-/// of all eighteen on average.
+/// Eight of 25 that were measured over the prefill's GEMMs (both models' four matrices and 14 more,
+/// 1 to 8192 rows, every K split): with these eight the best choice per GEMM is within 0.5 % of the
+/// best of the 14 shapes measured last on average.
 #define MUYO_GEMM_TILES(X)         \
     X(0, 4, 2, 1, 2, 4, 3, 32, 1)  \
     X(1, 2, 2, 2, 2, 3, 2, 64, 1)  \
-    X(2, 2, 4, 1, 1, 2, 3, 64, 1)  \
-    X(3, 2, 2, 2, 1, 3, 4, 64, 1)  \
-    X(4, 1, 2, 2, 1, 2, 3, 64, 2)  \
-    X(5, 1, 2, 4, 1, 2, 3, 128, 1) \
-    X(6, 1, 1, 4, 1, 2, 3, 128, 1)
+    X(2, 2, 4, 1, 2, 2, 3, 32, 1)  \
+    X(3, 2, 4, 1, 1, 2, 3, 64, 1)  \
+    X(4, 2, 2, 2, 1, 3, 4, 64, 1)  \
+    X(5, 1, 2, 2, 1, 2, 3, 64, 2)  \
+    X(6, 1, 2, 4, 1, 2, 3, 128, 1) \
+    X(7, 1, 1, 4, 1, 2, 3, 128, 1)
 
 /// What the choice of a shape needs to know. slabUs is the time of 64 columns of K with the CUs
 /// busy, tileUs what a round of tiles costs besides (first loads, epilogue), both fitted to those
-/// measurements.
+/// measurements. `margin` is above 1 for the shapes without sums for the lo products, which round
+/// twice as often: they are taken where they gain more than that.
 struct GemmTileCost
 {
     uint32_t bm, bn, bk, stages, perCu;
-    double slabUs, tileUs;
+    double slabUs, tileUs, margin;
 };
 
 constexpr GemmTileCost kGemmTiles[] = {
-    {256, 256, 32, 3, 1, 2.70, 9.8}, {128, 192, 64, 2, 1, 1.57, 3.5}, {64, 256, 64, 3, 1, 0.875, 2.4},
-    {64, 192, 64, 4, 1, 0.69, 3.4},  {32, 128, 64, 3, 2, 0.67, 1.4},  {32, 128, 128, 3, 1, 0.354, 2.5},
-    {32, 64, 128, 3, 1, 0.287, 2.4},
+    {256, 256, 32, 3, 1, 2.547, 0.01, 1.12}, {128, 192, 64, 2, 1, 1.495, 0.17, 1.03},
+    {128, 256, 32, 3, 1, 1.753, 0.01, 1.0},  {64, 256, 64, 3, 1, 0.941, 0.02, 1.0},
+    {64, 192, 64, 4, 1, 0.744, 0.72, 1.0},   {32, 128, 64, 3, 2, 0.756, 0.08, 1.0},
+    {32, 128, 128, 3, 1, 0.380, 2.05, 1.0},  {32, 64, 128, 3, 1, 0.292, 2.03, 1.0},
 };
 constexpr int kGemmTileCount = sizeof(kGemmTiles) / sizeof(kGemmTiles[0]);
 constexpr uint32_t kCus = 256;
@@ -516,11 +524,31 @@ uint32_t ColumnsPerSplit(uint32_t k, uint32_t splits)
     return CeilDiv(CeilDiv(k, kGemmSplitUnit), splits) * kGemmSplitUnit;
 }
 
-/// Estimated us of a launch of `tile` over `splits` K splits, with the partial planes' cost at
-/// their consumer: the rounds of resident workgroups times their slabs, or the time the weights
-/// take to arrive with the bytes each round keeps in flight (2 us each, at most 6 TB/s), whichever
-/// is longer. It ranks the shapes: over the measured GEMMs (88 with their own choice of splits, 88
-/// unsplit) the chosen one was 1.3 % slower than the fastest on average, 20 % at most.
+/// Token tiles of a group of GemmOrder. Over several rounds an XCD's 32 CUs hold about as many rows of
+/// both planes as of weights, in groups of about the same size. In a single round all tiles are
+/// resident, and an XCD's eighth of them is left in whole columns or rows of tiles: every token tile
+/// in one group, or one to a group where the activations are the larger operand (32 x 128 tiles, us,
+/// groups by the rule above / so: 513 rows of gate+up 2000 x 1784 26.8 / 21.9, 1500 rows of
+/// 896 x 4864 46.5 / 44.7, 1300 rows of 1000 x 1784 27.8 / 25.1).
+uint32_t GroupTiles(const GemmTileCost& tile, uint32_t rows, uint32_t n, uint32_t splits)
+{
+    const uint32_t mTiles = CeilDiv(rows, tile.bm);
+    if (static_cast<uint64_t>(mTiles) * CeilDiv(n, tile.bn) * splits <= kCus * tile.perCu)
+    {
+        return static_cast<uint64_t>(rows) * 2 <= n ? mTiles : 1;
+    }
+    const double most = std::round(std::sqrt(kCus / 8.0 * tile.perCu * tile.bn / (2.0 * tile.bm)));
+    return CeilDiv(mTiles, CeilDiv(mTiles, static_cast<uint32_t>(most)));
+}
+
+/// Estimated us of a launch of `tile` over `splits` K splits: the rounds of resident workgroups
+/// times their slabs, or the time the weights take to arrive with the bytes each round keeps in
+/// flight (1.52 us each, at most 9 TB/s), whichever is longer; the result's way to memory; and with
+/// splits the partial planes' and their consumer's. It ranks the shapes: over the measured GEMMs
+/// (unsplit with weights in cache and from memory, split with weights from memory, as a prompt's
+/// layers find them) the chosen one was 0.7 % slower than the fastest of the eight on average, 15 %
+/// at most. (Fitted with weights in cache alone, it left long K unsplit at 800 rows: 896 x 4864
+/// 24.4 us there, 33.9 in a prompt, where three splits take 25.4.)
 double GemmCost(const GemmTileCost& tile, uint32_t rows, uint32_t n, uint32_t k, uint32_t splits)
 {
     const double tiles = static_cast<double>(CeilDiv(rows, tile.bm)) * CeilDiv(n, tile.bn) * splits;
@@ -529,13 +557,30 @@ double GemmCost(const GemmTileCost& tile, uint32_t rows, uint32_t n, uint32_t k,
     const double last = tiles - fullRounds * slots;
     const double rounds = fullRounds + (last > 0.0 ? 1.0 : 0.0);
     const double slabs = std::min(CeilDiv(k, 64), ColumnsPerSplit(k, splits) / 64);
-    const double alone = tile.perCu > 1 && tiles <= kCus ? 0.6 : 1.0;  // a CU's workgroups slow one another
+    // A CU's workgroups slow one another: in one round, as many as meet another.
+    const double shared = fullRounds > 0.0 ? 1.0 : std::max(tiles - kCus, 0.0) / kCus;
+    const double slow = tile.perCu > 1 ? 0.98 + 0.02 * shared : 1.0;
     const double tileBytes = 2.0 * n * k / tiles;
     const double inFlight = static_cast<double>(tile.stages - 1) * tile.bn * tile.bk * 2;
-    auto arrive = [&](double count) { return count * tileBytes / std::min(6.0e6, count * inFlight / 2.0); };
+    auto arrive = [&](double count) { return count * tileBytes / std::min(9.09e6, count * inFlight / 1.52); };
     const double weights = fullRounds * arrive(slots) + (last > 0.0 ? arrive(last) : 0.0);
-    const double partial = splits > 1 ? 1.0 + 12.0 * splits * rows * n / 4.0e6 : 0.0;
-    return 2.0 + std::max(rounds * (slabs * tile.slabUs * alone + tile.tileUs), weights + tile.tileUs) + partial;
+    const double us = std::max(rounds * (slabs * tile.slabUs * slow + tile.tileUs), weights + tile.tileUs);
+    const double values = static_cast<double>(rows) * n / 1.0e6;
+    return tile.margin * (2.0 + us + 1.70 * values) + (splits > 1 ? 14.57 / 4.0 * splits * values : 0.0);
+}
+
+/// The fastest shape by that estimate.
+int BestTile(uint32_t rows, uint32_t n, uint32_t k, uint32_t splits)
+{
+    int best = 0;
+    for (int i = 1; i < kGemmTileCount; ++i)
+    {
+        if (GemmCost(kGemmTiles[i], rows, n, k, splits) < GemmCost(kGemmTiles[best], rows, n, k, splits))
+        {
+            best = i;
+        }
+    }
+    return best;
 }
 
 template <typename Epi>
@@ -546,17 +591,9 @@ hipError_t LaunchGemm(hipStream_t s, const uint16_t* ahi, const uint16_t* alo, c
     {
         return hipErrorInvalidValue;
     }
-    int best = 0;
-    for (int i = 1; i < kGemmTileCount; ++i)
-    {
-        if (GemmCost(kGemmTiles[i], rows, virtualRows, k, splits) < GemmCost(kGemmTiles[best], rows, virtualRows, k, splits))
-        {
-            best = i;
-        }
-    }
-    // The larger operand's tiles are the slower dimension of the order.
-    const bool mFast = static_cast<uint64_t>(rows) * 4 <= static_cast<uint64_t>(virtualRows) * 2;
-    const GemmOrder order{CeilDiv(rows, kGemmTiles[best].bm), CeilDiv(virtualRows, kGemmTiles[best].bn), mFast};
+    const int best = BestTile(rows, virtualRows, k, splits);
+    const GemmOrder order{CeilDiv(rows, kGemmTiles[best].bm), CeilDiv(virtualRows, kGemmTiles[best].bn),
+                          GroupTiles(kGemmTiles[best], rows, virtualRows, splits)};
     const uint64_t blocks = static_cast<uint64_t>(order.mTiles) * order.nTiles * splits;
     if (blocks > std::numeric_limits<int32_t>::max())
     {
@@ -570,7 +607,8 @@ hipError_t LaunchGemm(hipStream_t s, const uint16_t* ahi, const uint16_t* alo, c
     {                                                                                                                  \
         using T = GemmTile<WM, WN, WK, MB, NB, ST, BK, PER>;                                                           \
         static_assert(T::kBm == kGemmTiles[I].bm && T::kBn == kGemmTiles[I].bn && BK == kGemmTiles[I].bk &&            \
-                          ST == kGemmTiles[I].stages && PER == kGemmTiles[I].perCu,                                    \
+                          ST == kGemmTiles[I].stages && PER == kGemmTiles[I].perCu &&                                  \
+                          T::kLowSums == (kGemmTiles[I].margin == 1.0),                                                \
                       "kGemmTiles");                                                                                   \
         hipLaunchKernelGGL((GemmSplitKernel<T, WM, WN, WK, MB, NB, ST, BK, Epi>), dim3(static_cast<uint32_t>(blocks)), \
                            dim3(T::kThreads), 0, s, ahi, alo, epi, rows, k, kPerSplit, order);                         \
@@ -596,14 +634,11 @@ uint32_t GemmSplits(uint32_t rows, uint32_t n, uint32_t k)
         {
             continue;
         }
-        for (const GemmTileCost& tile : kGemmTiles)
+        const double cost = GemmCost(kGemmTiles[BestTile(rows, n, k, splits)], rows, n, k, splits);
+        if (cost < bestCost)
         {
-            const double cost = GemmCost(tile, rows, n, k, splits);
-            if (cost < bestCost)
-            {
-                bestCost = cost;
-                best = splits;
-            }
+            bestCost = cost;
+            best = splits;
         }
     }
     return best;
@@ -635,3 +670,17 @@ hipError_t LaunchGemmSwiGlu(hipStream_t s, const uint16_t* ahi, const uint16_t* 
     return LaunchGemm(s, ahi, alo, SwiGluEpi{wgate, wup, hhi, hlo, ffn, k}, rows, virtualRows, k);
 }
 }  // namespace muyo
+
+// For the tests (no device needed): the tile (tokens, weight rows, columns of a slab), token tiles
+// per group, and K splits of a launch; splits 0 for the decoder's choice of them. For the swiglu
+// GEMM n is twice the outputs, in whole 32s.
+extern "C" void muyo_prefill_gemm_plan(uint32_t rows, uint32_t n, uint32_t k, uint32_t splits, uint32_t plan[5])
+{
+    const uint32_t z = splits > 0 ? splits : muyo::GemmSplits(rows, n, k);
+    const muyo::GemmTileCost& tile = muyo::kGemmTiles[muyo::BestTile(rows, n, k, z)];
+    plan[0] = tile.bm;
+    plan[1] = tile.bn;
+    plan[2] = tile.bk;
+    plan[3] = muyo::GroupTiles(tile, rows, n, z);
+    plan[4] = z;
+}

@@ -221,21 +221,25 @@ def test_gemm_swiglu_matches_per_token_path(mh, gpu, orc, rows, ffn, k):
     assert worst(got, want) < 2e-5
 
 
-# Each tile shape of the GEMM at a size that selects it, one past a whole tile in rows or weight
-# rows, with a K that ends inside a slab and inside a 16-column step.
+# Each tile shape of the GEMM (tokens, weight rows, columns of a slab; test_prefill_plan.py holds the
+# choice to it, for the swiglu GEMM of n outputs' worth of weight rows too) at a size a little past
+# whole tiles in rows and weight rows, with a K that ends inside a slab and inside a 16-column step.
 TILE_SHAPES = [
-    (980, 13420, 264),   # 256 x 256
-    (208, 21076, 264),   # 128 x 192
-    (1541, 1364, 264),   # 64 x 256
-    (1, 33592, 536),     # 64 x 192
-    (65, 9732, 280),     # 32 x 128, two workgroups per CU
-    (33, 9092, 904),     # 32 x 128, 128-column slabs
-    (33, 132, 584),      # 32 x 64
-    (1, 4, 8),
+    (1290, 10264, 280, (256, 256, 32)),
+    (641, 7108, 248, (128, 192, 64)),
+    (133, 27916, 200, (128, 256, 32)),
+    (69, 31260, 200, (64, 256, 64)),
+    (1541, 1364, 264, (64, 192, 64)),   # one round of workgroups, a token tile to a group
+    (1541, 5000, 520, (64, 256, 64)),   # two rounds, groups of seven token tiles, the last of four
+    (321, 5964, 648, (64, 192, 64)),
+    (65, 9732, 280, (32, 128, 64)),     # two workgroups per CU
+    (33, 9092, 904, (32, 128, 128)),
+    (33, 132, 584, (32, 64, 128)),
+    (1, 4, 8, (32, 128, 64)),
 ]
 
 
-@pytest.mark.parametrize("rows,n,k", TILE_SHAPES)
+@pytest.mark.parametrize("rows,n,k", [case[:3] for case in TILE_SHAPES])
 def test_gemm_tile_shapes_exact_with_both_planes(mh, gpu, rows, n, k):
     """Values whose products and sums are exact in f32 (hi and weights integers up to 2, lo a
     multiple of 2^-11 up to 2^-10: sums below 2^12 in steps of 2^-11, 23 bits), so the plain GEMM must

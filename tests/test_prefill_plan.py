@@ -4,7 +4,7 @@ import ctypes
 
 import pytest
 
-from test_prefill_gpu import CHUNK_CASES
+from test_prefill_gpu import CHUNK_CASES, TILE_SHAPES
 
 
 @pytest.fixture(scope="module")
@@ -61,3 +61,70 @@ def test_attention_chunks_of_small_merges(attention_plan, rows, pos0, chunks):
 def test_attention_chunk_cases_are_planned_as_they_say(attention_plan, heads, kv_heads, head_dim, rows, pos0, max_seq,
                                                        check, planned):
     assert attention_plan(heads, kv_heads, head_dim, rows, pos0)[:2] == planned
+
+
+@pytest.fixture(scope="module")
+def gemm_plan(mh):
+    call = ctypes.CDLL(str(mh.LIB_PATH)).muyo_prefill_gemm_plan
+    call.restype = None
+
+    def plan(rows, n, k, splits=1):
+        """(tokens, weight rows, slab columns) of the tile, token tiles per group, K splits (0: chosen)."""
+        out = (ctypes.c_uint32 * 5)()
+        call(rows, n, k, splits, out)
+        return tuple(out[:3]), out[3], out[4]
+
+    return plan
+
+
+@pytest.mark.parametrize("rows,n,k,tile", TILE_SHAPES)
+def test_gemm_tile_cases_take_the_tiles_they_say(gemm_plan, rows, n, k, tile):
+    assert gemm_plan(rows, n, k)[0] == tile
+    ffn = n // 8 * 4 or 4
+    assert gemm_plan(rows, -(-ffn // 16) * 32, k)[0] == tile
+
+
+def test_gemm_tile_cases_cover_every_tile(gemm_plan):
+    covered = {case[3] for case in TILE_SHAPES}
+    for rows in (1, 7, 33, 64, 100, 200, 301, 613, 900, 1300, 1500, 2048, 4096, 8192):
+        for n in (64, 896, 1152, 2560, 3584, 4608, 9728, 37888, 151936):
+            for k in (64, 896, 3584, 4864, 18944):
+                assert gemm_plan(rows, n, k)[0] in covered, (rows, n, k)
+
+
+# The fastest measured tile, or one within 2 % of it, at full prompts of both widths, an ordinary one, a
+# short turn and some other large products.
+@pytest.mark.parametrize("rows,n,k,tile", [
+    (2048, 9728, 896, (64, 256, 64)), (4096, 9728, 896, (128, 256, 32)), (2048, 37888, 3584, (256, 256, 32)),
+    (2048, 3584, 3584, (128, 256, 32)), (2048, 3584, 18944, (128, 256, 32)), (2048, 28672, 4096, (256, 256, 32)),
+    (8192, 151936, 896, (256, 256, 32)), (613, 9728, 896, (128, 192, 64)), (301, 896, 4864, (32, 64, 128)),
+    (45, 37888, 3584, (64, 192, 64)),
+])
+def test_gemm_takes_the_measured_tile(gemm_plan, rows, n, k, tile):
+    assert gemm_plan(rows, n, k)[0] == tile
+
+
+def test_gemm_groups_of_token_tiles(gemm_plan):
+    """Over several rounds of workgroups, near the square of an XCD's resident tiles and all of about the
+    same size; in one round all token tiles, or one where there are more of them than weight rows."""
+    for rows, n, k, tile, group in ((8192, 28672, 4096, 256, 4), (2048, 37888, 3584, 256, 4), (2048, 9728, 896, 64, 8),
+                                    (1541, 5000, 520, 64, 7), (45, 37888, 3584, 64, 1), (513, 2000, 1784, 32, 17),
+                                    (1500, 896, 4864, 32, 1), (301, 9728, 896, 64, 5)):
+        assert gemm_plan(rows, n, k)[0][0] == tile, (rows, n, k)
+        assert gemm_plan(rows, n, k)[1] == group, (rows, n, k)
+
+
+def test_gemm_splits_give_every_split_work(gemm_plan):
+    """Whole 128-column units per split, none empty; at most eight up to 512 rows, four beyond, which is
+    what the decoder's partial planes are sized for. The prompts of the decoder's tests meet one, a
+    few and more than four splits (the norm and rope kernels sum up to one, four or eight)."""
+    seen = set()
+    for rows in (1, 24, 40, 96, 300, 301, 512, 513, 1024, 1990, 2048):
+        for n, k in ((1152, 896), (896, 896), (896, 4864), (4608, 3584), (3584, 3584), (3584, 18944), (512, 256), (64, 8)):
+            splits = gemm_plan(rows, n, k, 0)[2]
+            units = -(-k // 128)
+            assert 1 <= splits <= (8 if rows <= 512 else 4)
+            assert -(-units // -(-units // splits)) == splits, (rows, n, k)
+            if (n, k) in ((1152, 896), (896, 4864)) and rows in (96, 300):
+                seen.add(splits)
+    assert min(seen) <= 3 and max(seen) > 4
