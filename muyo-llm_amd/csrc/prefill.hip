@@ -1,6 +1,6 @@
-// Batched-prefill kernels for gfx950: a causal flash attention over the fp16 cache and the row-wise
-// glue (embedding, rms_norm into split planes, rope + cache append). The GEMMs are in
-// prefill_gemm.hip.
+// Batched-prefill kernels for gfx950: the row-wise glue (embedding, rms_norm into split planes,
+// rope + cache append) and the entry points of all of them. The GEMMs are in prefill_gemm.hip, the
+// attention in prefill_attention.hip.
 #include <algorithm>
 #include <cmath>
 #include <initializer_list>
@@ -111,9 +111,9 @@ __global__ __launch_bounds__(256) void RmsNormSplitKernel(float* __restrict__ x,
 }
 
 /// RmsNormSplitKernel with kT threads per row (one wave, or the whole 256-thread workgroup) and
-/// at most kChunks 16-byte chunks of the row per thread (and kParts K splits), all requested before the first is used:
-/// every K split's part, the residual and the weight in one round of loads instead of one round
-/// per chunk. The sums run in SplitSum::At's order; the sum of squares meets across the row's
+/// at most kChunks 16-byte chunks of the row per thread (and kParts K splits), all requested before
+/// the first is used: every K split's part, the residual and the weight in one round of loads
+/// instead of one round per chunk. The sums run in SplitSum::At's order; the sum of squares meets across the row's
 /// waves in LDS.
 template <int kT, uint32_t kParts>
 __global__ __launch_bounds__(256) void RmsNormSplitRowsKernel(float* __restrict__ x, const float* __restrict__ w,

@@ -521,11 +521,11 @@ struct ArgMaxArgs
     uint32_t gx, gy, gz;
 };
 
-/// One row by a workgroup of kThreads, each with kDepth 16-byte loads in flight. With a workgroup per
-/// CU or fewer, nothing else hides a row's latency: 256 threads of four loads (16 KB in flight) take
-/// 38 round trips over a row of 151936, 20.1 us where the LM head has just written it; 1024 threads
-/// of eight take five, about 10 us. Batches of many rows keep the small workgroups, whose number
-/// hides it. (Splitting a row over workgroups without a workspace, each exchanging its index into d
+/// One row by a workgroup of kThreads, each with up to kDepth 16-byte loads in flight. With a workgroup
+/// per CU or fewer, nothing else hides a row's latency: 256 threads of four loads (16 KB in flight)
+/// take 38 round trips over a row of 151936, 20.1 us where the LM head has just written it; 1024
+/// threads of eight take four, and six of one load for what is left of the row, about 10 us.
+/// Batches of many rows keep the small workgroups, whose number hides it. (Splitting a row over workgroups without a workspace, each exchanging its index into d
 /// atomically, took 7.1 us for one row but 45 against 20 for 64: the exchanges queue.)
 template <int kThreads, int kDepth>
 __global__ __launch_bounds__(kThreads) void ArgMaxRows(const float* __restrict__ a, int32_t* __restrict__ d,
