@@ -148,8 +148,8 @@ __device__ constexpr int KeyOf(int r) { return 32 * (r / 16) + 8 * (r % 16 / 4) 
 /// rises by 2^8 (head_dim 128: 300 vector instructions per 32 keys before, about 150 since) or by
 /// the multiply-add that takes in a step's sum (64). Measured, before (one 32-key tile in LDS, V
 /// transposed by hand, a barrier pair per tile) and now, us: 28 / 4 heads of 128, 777 rows after
-/// 5003: 348 / 150; 2048 rows 142 / 88; 45 rows after 700: 38 / 14.6; 14 / 2 heads of 64, 613 rows
-/// 28.6 / 14.9, 2048 rows 53 / 42.
+/// 5003: 348 / 150; 2048 rows 142 / 92; 45 rows after 700: 38 / 14.6; 14 / 2 heads of 64, 613 rows
+/// 28.6 / 14.9, 2048 rows 53 / 45.
 ///
 /// Grid: kv heads fastest (an XCD then sees one or two of them), then pairs, the longest first, then
 /// key chunks: whole chunks start before the tails, and an XCD does not get one chunk of every
